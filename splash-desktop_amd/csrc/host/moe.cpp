@@ -295,32 +295,59 @@ void MoE::addRouted(hipStream_t graph, const MoeBuffers &b, const MoeWeights &w,
     const uint64_t tiles = uint64_t{s.sharedSlices} * ((plan.rows() + plan.tileRows() - 1) / plan.tileRows());
     return mode == 1 && plan.tileRows() > 16 && tiles * (outputSize / 64) <= 2 * kern::kPrefillUnits ? 1 : 0;
   };
-  launches(gateUpFormats, [&](uint32_t mode, uint32_t gateFormat, uint32_t upFormat) {
-    a.mode = mode;
-    a.row_halves = halves(mode, s.expertIntermediateSize);
-    if (gateFormat == upFormat) {
-      bind(0, w.gate, w.sharedGate);
-      bind(1, w.up, w.sharedUp);
-      a.fmt = gateFormat;
-      a.gate_up = 1;
-      a.gate = nullptr;
-      a.output = sc.expertIntermediate.as<uint16_t>();
-      launched(kern::launch_moe_expert(a, graph), "MoE gate/up pass");
-      return;
-    }
-    a.gate_up = 0;
+  // The 8-row tiles of decode steps and the smallest chunks run one launch a pass, routed and shared tiles each in
+  // their own format.
+  const bool small = plan.tileRows() <= 16;
+  const auto runSmall = [&](uint32_t routedFormat, uint32_t sharedFormat, const char *what) {
+    a.mode = 2;
+    a.fmt = routedFormat;
+    a.shared_fmt = s.sharedSlices ? sharedFormat : routedFormat;
+    launched(kern::launch_moe_expert_small(a, graph), what);
+  };
+  if (small && w.gate.formatId == w.up.formatId &&
+      (!s.sharedSlices || w.sharedGate.formatId == w.sharedUp.formatId)) {
+    bind(0, w.gate, w.sharedGate);
+    bind(1, w.up, w.sharedUp);
+    a.gate_up = 1;
+    a.output = sc.expertIntermediate.as<uint16_t>();
+    runSmall(w.gate.formatId, w.sharedGate.formatId, "MoE gate/up pass");
+  } else if (small) {
     bind(0, w.gate, w.sharedGate);
     bind(1, none, none);
-    a.fmt = gateFormat;
-    a.gate = nullptr;
     a.output = sc.expertOutput.as<uint16_t>();
-    launched(kern::launch_moe_expert(a, graph), "MoE gate pass");
+    runSmall(w.gate.formatId, w.sharedGate.formatId, "MoE gate pass");
     bind(0, w.up, w.sharedUp);
-    a.fmt = upFormat;
     a.gate = sc.expertOutput.as<const uint16_t>();
     a.output = sc.expertIntermediate.as<uint16_t>();
-    launched(kern::launch_moe_expert(a, graph), "MoE up pass");
-  });
+    runSmall(w.up.formatId, w.sharedUp.formatId, "MoE up pass");
+  } else {
+    launches(gateUpFormats, [&](uint32_t mode, uint32_t gateFormat, uint32_t upFormat) {
+      a.mode = mode;
+      a.row_halves = halves(mode, s.expertIntermediateSize);
+      if (gateFormat == upFormat) {
+        bind(0, w.gate, w.sharedGate);
+        bind(1, w.up, w.sharedUp);
+        a.fmt = gateFormat;
+        a.gate_up = 1;
+        a.gate = nullptr;
+        a.output = sc.expertIntermediate.as<uint16_t>();
+        launched(kern::launch_moe_expert(a, graph), "MoE gate/up pass");
+        return;
+      }
+      a.gate_up = 0;
+      bind(0, w.gate, w.sharedGate);
+      bind(1, none, none);
+      a.fmt = gateFormat;
+      a.gate = nullptr;
+      a.output = sc.expertOutput.as<uint16_t>();
+      launched(kern::launch_moe_expert(a, graph), "MoE gate pass");
+      bind(0, w.up, w.sharedUp);
+      a.fmt = upFormat;
+      a.gate = sc.expertOutput.as<const uint16_t>();
+      a.output = sc.expertIntermediate.as<uint16_t>();
+      launched(kern::launch_moe_expert(a, graph), "MoE up pass");
+    });
+  }
   // Down over the grouped intermediate rows.
   a.input = sc.expertIntermediate.as<const uint16_t>();
   a.routes = nullptr;
@@ -335,12 +362,16 @@ void MoE::addRouted(hipStream_t graph, const MoeBuffers &b, const MoeWeights &w,
   const auto downFormats = [&](uint32_t mode) {
     return std::pair{mode == 0 ? w.down.formatId : w.sharedDown.formatId, 0u};
   };
-  launches(downFormats, [&](uint32_t mode, uint32_t format, uint32_t) {
-    a.mode = mode;
-    a.row_halves = halves(mode, s.hiddenSize);
-    a.fmt = format;
-    launched(kern::launch_moe_expert(a, graph), "MoE down pass");
-  });
+  if (small) {
+    runSmall(w.down.formatId, w.sharedDown.formatId, "MoE down pass");
+  } else {
+    launches(downFormats, [&](uint32_t mode, uint32_t format, uint32_t) {
+      a.mode = mode;
+      a.row_halves = halves(mode, s.hiddenSize);
+      a.fmt = format;
+      launched(kern::launch_moe_expert(a, graph), "MoE down pass");
+    });
+  }
   const SqMoeCombineParams combine{plan.rows(), s.hiddenSize, s.routesPerToken()};
   launched(kern::launch_moe_combine(sc.expertOutput.as<const uint16_t>(), sc.routeRows.as<const uint32_t>(),
                                     sc.routingWeights.as<const float>(), b.residual.as<const uint16_t>(),

@@ -382,7 +382,7 @@ __device__ __forceinline__ void expert_tile(const MoeExpertArgs &a, SqMoeTileDes
   // gate/up pair only moves more of its MFMA results through the accumulation registers. Short chunks fit more
   // waves a SIMD (expert_kernel), and each resident wave covers more of the others' dependency stalls.
   constexpr bool kShort = short_chunks<FMT, NT>();
-  row_stream<FMT, MB, NT, 2, kShort ? 2 : 4, !kShort>(plane, high, meta, xrow, G, acc);
+  row_stream<FMT, MB, NT, 2, kShort ? 2 : 4, !kShort>(plane, high, meta, xrow, 0, G, acc);
   // Column 16 t + j of the tile: the gathering passes store it at its place in the read order (chunk 4 g + j / 4 of
   // group g = 2 ct + t / 2, then position 4 (t % 2) + j % 4), for the down pass; the down pass in column order.
   const uint32_t column = a.gather ? 8 * (j >> 2) + (j & 3) : j;
@@ -478,6 +478,82 @@ void expert_kernel(MoeExpertArgs a) {
   else expert_tile<FMT, MB, NT>(a, d, tile, ct, 0, d.rows);
 }
 
+// Wave `slice`'s groups of tensor slot n of column tile ct against the at most 16 rows of a small tile, into acc.
+template <uint32_t FMT>
+__device__ __forceinline__ void small_walk(const MoeExpertArgs &a, SqMoeTileDescriptor d, uint32_t first_row, int n,
+                                           uint32_t ct, uint32_t slice, float (&acc)[1][4][1][4]) {
+  using F = Fmt<FMT>;
+  const int lane = threadIdx.x & 63, j = lane & 15, q = lane >> 4;
+  const uint32_t G = a.K >> 5, spans = (G + 3) / 4;
+  const uint32_t first = spans * slice / a.slices * 4, end = min(G, spans * (slice + 1) / a.slices * 4);
+  if (first >= end) return;
+  const bool shared = d.expert >= a.experts;
+  const size_t pt = (size_t)(shared ? d.expert - a.experts : a.slots[d.expert]) * (a.output_size / 64) + ct;
+  const uint8_t *const plane[1] = {(shared ? a.shared_plane0[n] : a.plane0[n]) + (pt * G * 64 + lane) * F::P0};
+  const uint8_t *const high[1] = {
+      F::P1 ? (shared ? a.shared_plane1[n] : a.plane1[n]) + (pt * G * 64 + lane) * F::P1 : nullptr};
+  const uint8_t *const meta[1] = {(shared ? a.shared_meta[n] : a.meta[n]) + (pt * (G / F::UNIT) * 64 + lane) * F::META};
+  const uint32_t r = (uint32_t)j < d.rows ? j : 0u;
+  const uint32_t source = a.gather ? a.routes[first_row + r] / a.routes_per_row : first_row + r;
+  const uint16_t *const xrow[1] = {a.input + (size_t)source * a.K + 8 * q};
+  row_stream<FMT, 1, 1, 2, F::P0 == 32 || F::P1 ? 2 : 4, false>(plane, high, meta, xrow, first, end, acc);
+}
+
+// The expert passes of 8-row tiles (decode steps and the smallest chunks: an expert's one to eight rows). There are
+// few tiles and each wave's walk over K is a chain of loads it waits on, so K is cut into `slices` slices, a wave each,
+// and a gate/up pass gives gate and up waves of their own: a workgroup's eight waves are the slices of the tensors of
+// 8 / (slices x tensors) column tiles, their sums meet in LDS in slice order. One launch runs the routed and the shared
+// tiles, each in its own format, so that the shared slices' long chains overlap the routed ones. 128 registers a wave
+// (chunks of two groups for the formats of more bits), so that two workgroups share a compute unit. Measured, 8 rows
+// over 256 experts of 2048 x 512 (Q4_K gate/up, Q5_K down, a Q8_0 shared slice): gate/up 40.6 us routed and 62.5 us
+// shared in two launches of whole-K waves -> 25 us; down 17.1 and 10.2 -> 17.5; at 170 registers 33 and 24.
+constexpr uint32_t kSmallWaves = 8;
+__global__ __launch_bounds__(64 * kSmallWaves) __attribute__((amdgpu_waves_per_eu(4)))
+void expert_small_kernel(MoeExpertArgs a) {
+  const uint32_t tile = blockIdx.y;
+  if (tile >= a.tile_count->tiles) return;
+  const SqMoeTileDescriptor d = a.tiles[tile];
+  const int lane = threadIdx.x & 63, j = lane & 15, q = lane >> 4;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), tensors = a.gate_up ? 2 : 1;
+  const uint32_t per = kSmallWaves / (a.slices * tensors), ct0 = blockIdx.x * per;
+  const uint32_t column = wave / (a.slices * tensors), n = wave / a.slices % tensors, slice = wave % a.slices;
+  const uint32_t column_tiles = a.output_size / 64, first_row = tile * a.tile_rows;
+  float acc[1][4][1][4];
+  clear(acc);
+  if (ct0 + column < column_tiles) {
+    const uint32_t fmt = d.expert >= a.experts ? a.shared_fmt : a.fmt;
+    with_format(fmt, [&](auto f) { small_walk<decltype(f)::value>(a, d, first_row, n, ct0 + column, slice, acc); });
+  }
+  // red[wave][4 t + i][lane]: column block t, row 4 q + i.
+  __shared__ float red[kSmallWaves][16][64];
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) red[wave][4 * t + i][lane] = acc[0][t][0][i];
+  __syncthreads();
+  const auto total = [&](uint32_t from, uint32_t f) __attribute__((always_inline)) {
+    float v = 0.0f;
+    for (uint32_t s = 0; s < a.slices; ++s) v += red[from + s][f][lane];
+    return v;
+  };
+  for (uint32_t o = wave; o < per * 16; o += kSmallWaves) {
+    const uint32_t c = o / 16, f = o % 16, ct = ct0 + c, r = 4u * q + (f & 3), t = f >> 2;
+    if (ct >= column_tiles || r >= d.rows) continue;
+    // The gathering passes store in the read order, the down pass in column order (expert_tile).
+    const uint32_t place = a.gather ? 32 * (t >> 1) + 4 * (t & 1) + 8 * (j >> 2) + (j & 3) : 16 * t + j;
+    const size_t at = (size_t)(first_row + r) * a.output_size + ct * 64 + place;
+    const uint32_t from = c * a.slices * tensors;
+    float v = total(from, f);
+    if (a.gate_up) {
+      const float u = bf16_to_f32(f32_to_bf16(total(from + a.slices, f)));
+      v = u * silu(bf16_to_f32(f32_to_bf16(v)));
+    } else if (a.gate) {
+      v = bf16_to_f32(f32_to_bf16(v)) * silu(bf16_to_f32(a.gate[at]));
+    }
+    a.output[at] = f32_to_bf16(v);
+  }
+}
+
 // Thread: one 16-byte chunk of the table, chunk c of a group of 32 inputs: its 4-input units c and c + 4 (inputs
 // 4c..4c+3 and 16+4c..19+4c, the group's dwords 2c, 2c + 1 and 8 + 2c, 9 + 2c), the prefill's half rows order
 // (half_rows.hpp). The reference's routed pass opens with its gather of the input rows into the grouped input
@@ -564,7 +640,7 @@ hipError_t launch_expert_rows(const MoeExpertArgs &a, hipStream_t stream) {
 template <uint32_t FMT>
 hipError_t launch_expert_format(const MoeExpertArgs &a, hipStream_t stream) {
   const bool pairs = affine4_short<FMT>() && !a.gate_up && !a.gather && (a.output_size / 64) % 2 == 0;
-  if (a.tile_rows <= 16 || a.row_halves)
+  if (a.row_halves)
     return a.gate_up || pairs ? launch_expert_rows<FMT, 1, 2>(a, stream) : launch_expert_rows<FMT, 1, 1>(a, stream);
   return a.gate_up || pairs ? launch_expert_rows<FMT, 2, 2>(a, stream) : launch_expert_rows<FMT, 2, 1>(a, stream);
 }
@@ -597,7 +673,20 @@ hipError_t launch_moe_input_rows(const uint16_t *input, uint32_t rows, uint32_t 
   return hipGetLastError();
 }
 
+hipError_t launch_moe_expert_small(const MoeExpertArgs &args, hipStream_t stream) {
+  if (args.tile_rows > 16 || !args.max_tiles) return hipErrorInvalidValue;
+  MoeExpertArgs a = args;
+  // Slices of at least eight groups (the loads a wave keeps in flight) and at most four of them, in a power of two.
+  const uint32_t spans = a.K / 32 / 4;
+  a.slices = spans >= 8 ? 4 : spans >= 4 ? 2 : 1;
+  const uint32_t per = kSmallWaves / (a.slices * (a.gate_up ? 2 : 1));
+  hipLaunchKernelGGL(expert_small_kernel, dim3((a.output_size / 64 + per - 1) / per, a.max_tiles),
+                     dim3(64 * kSmallWaves), 0, stream, a);
+  return hipGetLastError();
+}
+
 hipError_t launch_moe_expert(const MoeExpertArgs &a, hipStream_t stream) {
+  if (a.tile_rows != 32) return hipErrorInvalidValue;
   switch (a.fmt) {
     case SQ_FMT_AF4G32: return launch_expert_format<SQ_FMT_AF4G32>(a, stream);
     case SQ_FMT_AF4G64: return launch_expert_format<SQ_FMT_AF4G64>(a, stream);

@@ -362,9 +362,10 @@ __device__ __forceinline__ void row_slice(const RowBuffers<FMT, NT, MB, TB> &src
   }
 }
 
-// Adds all G groups of NT tensors' plane tiles to acc, as row_slice does, in one continuous stream: chunks of CH
-// groups, each chunk's loads (clamped to the last group, so every chunk issues as many) issued SETS - 1 chunks
-// ahead into a ring of SETS register sets; AHEAD builds each group's operands a group ahead (else just before its
+// Adds groups first .. end - 1 of NT tensors' plane tiles to acc, as row_slice does, in one continuous stream: chunks
+// of CH groups, each chunk's loads (clamped to the last group, so every chunk issues as many) issued SETS - 1 chunks
+// ahead into a ring of SETS register sets; first is a multiple of CH and of the meta unit or lies CH-aligned inside a
+// longer one; AHEAD builds each group's operands a group ahead (else just before its
 // MFMAs). plane[n] and high[n] point at group 0 for the lane, meta[n] at unit 0 of the lane's own column l (one
 // load per unit and tensor, spread_coefs hands each lane the columns its MFMA blocks hold). The input rows come in the
 // tile's read order
@@ -374,11 +375,11 @@ __device__ __forceinline__ void row_slice(const RowBuffers<FMT, NT, MB, TB> &src
 template <uint32_t FMT, int MB, int NT, int SETS = 2, int CH = 4, bool AHEAD = true>
 __device__ __forceinline__ void row_stream(const uint8_t *const (&plane)[NT], const uint8_t *const (&high)[NT],
                                            const uint8_t *const (&meta)[NT], const uint16_t *const (&xrow)[MB],
-                                           uint32_t G, float (&acc)[NT][4][MB][4]) {
+                                           uint32_t first, uint32_t end, float (&acc)[NT][4][MB][4]) {
   using F = Fmt<FMT>;
   constexpr int SG = F::SG, UNIT = F::UNIT, MU = UNIT < CH ? CH / UNIT : 1;
   static_assert(CH % SG == 0, "a chunk holds whole scale groups");
-  const uint32_t last = G - 1, chunks = (G + CH - 1) / CH;
+  const uint32_t last = end - 1, chunks = (end - first + CH - 1) / CH;
   const CodeConstants cc = make_code_constants();
   const uint32_t hshift = row_high_shift<FMT>(threadIdx.x & 63);
   u32x4 xv[SETS][MB][CH];
@@ -387,7 +388,7 @@ __device__ __forceinline__ void row_stream(const uint8_t *const (&plane)[NT], co
   const auto issue = [&](uint32_t c, int set) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < CH; ++u) {
-      const uint32_t g = min(c * CH + u, last);
+      const uint32_t g = min(first + c * CH + u, last);
 #pragma unroll
       for (int b = 0; b < MB; ++b) xv[set][b][u] = *(const u32x4 *)(xrow[b] + (size_t)g * 32);
 #pragma unroll
@@ -395,7 +396,7 @@ __device__ __forceinline__ void row_stream(const uint8_t *const (&plane)[NT], co
     }
 #pragma unroll
     for (int m = 0; m < MU; ++m) {
-      const uint32_t unit = min((c * CH) / UNIT + m, last / UNIT);
+      const uint32_t unit = min((first + c * CH) / UNIT + m, last / UNIT);
 #pragma unroll
       for (int n = 0; n < NT; ++n) own[set][n][m] = load_meta<FMT>(meta[n] + (size_t)unit * 64 * F::META);
     }
@@ -414,9 +415,9 @@ __device__ __forceinline__ void row_stream(const uint8_t *const (&plane)[NT], co
   const auto compute = [&](uint32_t c, int set, int next_set) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < CH; ++u) {
-      const uint32_t g = c * CH + u;
-      const int os = kAhead ? u & 1 : 0;   // CH is even: group g's operands sit in set g % 2
-      if (g < G) {
+      const uint32_t g = first + c * CH + u;
+      const int os = kAhead ? u & 1 : 0;   // CH is even: group g's operands sit in set u % 2
+      if (g < end) {
         u32x4 x[MB];
 #pragma unroll
         for (int b = 0; b < MB; ++b) x[b] = xv[set][b][u];

@@ -229,6 +229,23 @@ def test_moe_routed_formats(fmt, rows):
     check_block(block, x, scores, 4, None, "prefill" if rows > 32 else "decode")
 
 
+@pytest.mark.parametrize("fmt,hidden,inner", [
+    (oracle.FMT_AF4G32, 256, 64),      # one slice, one column tile of a workgroup's four
+    (oracle.FMT_AF4G64, 1024, 576),    # four slices; a down of 18 groups: two, the last short of a span
+    (oracle.FMT_AF4G64, 768, 1088),    # three spans a slice pair; a down of 34 groups in four slices, the last short
+    (oracle.FMT_AF8G64, 1280, 320),    # spans that do not divide over the slices
+    (oracle.FMT_Q6K, 2048, 1024)])
+def test_moe_small_tile_slices(fmt, hidden, inner):
+    """The 8-row tiles' K slices: short last spans, column tiles short of a workgroup's, and routed and shared tiles of
+    two formats in one launch. The same bound as every block here."""
+    rng = np.random.default_rng(hidden + inner)
+    block = Block(rng, 12, hidden, inner, fmt=fmt, shared=1, gated=True, shared_fmt=oracle.FMT_AF4G64)
+    x = synthetic.activations(rng, 9, hidden)
+    scores = synthetic.router_logits(rng, 9, 12)
+    residual = synthetic.bf16_bits(rng.uniform(-2, 2, (9, hidden)).astype(np.float32))
+    check_block(block, x, scores, 3, residual, "decode")
+
+
 @pytest.mark.parametrize("rows,phase", [(48, "prefill"), (5, "decode")])
 def test_moe_projections_in_formats_of_their_own(rows, phase):
     """Every projection in its own format (MoE.cpp:27-62): a routed gate and up of different formats (a gate pass and
