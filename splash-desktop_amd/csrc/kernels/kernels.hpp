@@ -92,6 +92,14 @@ struct PrefillArgs {
   uint32_t stream_dp, stream_tiles, stream_range, stream_row_blocks;
 };
 hipError_t launch_prefill(uint32_t fmt, uint32_t epilogue, const PrefillArgs &args, hipStream_t stream);
+// The narrow tile's shape for a projection of `rows` x `plane_tiles` plane tiles (prefill_narrow.hip): 64 or 96 rows x 32
+// or 64 columns a workgroup; rows 0 where the wide tile (prefill.hip) runs. `split`: the wide tile would halve its K.
+struct PrefillNarrow {
+  uint32_t rows, columns;
+};
+PrefillNarrow prefill_narrow(uint32_t rows, uint32_t plane_tiles, uint32_t K, bool split);
+hipError_t launch_prefill_narrow(uint32_t fmt, uint32_t epilogue, const PrefillArgs &args, PrefillNarrow narrow,
+                                 hipStream_t stream);
 // The prefill dispatch's shape: tiles of bm rows (128 or 256) by four plane tiles, row_blocks x column_groups of
 // them, 64 inputs a step, one workgroup each. With `split` (prefill_split of the projection's rows, whole width and
 // K), the tiles from column group whole_groups on are cut at step split_at between two workgroups, which store their

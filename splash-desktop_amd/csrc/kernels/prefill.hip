@@ -956,6 +956,31 @@ PrefillSchedule prefill_schedule(uint32_t rows, uint32_t plane_tiles, uint32_t K
   if (7 * rounds128 < 10 * rounds256) return {128, 0, blocks128, columns, 0, 0};
   return {256, 0, blocks256, columns, 0, 0};
 }
+// The narrow tile's shape where its rounds of workgroups over the compute units cost less than the wide tile's, in
+// microseconds a 64-input step a round. Measured (Q4_K; the other formats' ratios are alike): 64 x 32 0.16-0.17, 64 x
+// 64 0.23-0.28, 96 x 32 0.21-0.23, 96 x 64 0.30-0.32 (128 x 32, 0.27-0.30, never costs less than 64 x 64); wide tiles
+// of 128 rows 1.03, of 256 1.87, halved 1.8 a step of a half and 15 for the close. The wide tile keeps what the narrow
+// one would not win by a twentieth. A function of the projection's whole width, so that every dispatch of it (one per
+// format) takes the same tile.
+PrefillNarrow prefill_narrow(uint32_t rows, uint32_t plane_tiles, uint32_t K, bool split) {
+  const double steps = K / BK;
+  const auto rounds = [&](uint32_t r, uint32_t c) {
+    return ((uint64_t)((rows + r - 1) / r) * ((plane_tiles * 64 + c - 1) / c) + kPrefillUnits - 1) / kPrefillUnits;
+  };
+  const double wide = split ? 0.9 * steps + 15.0
+                            : steps * std::min(1.03 * (double)rounds(128, 256), 1.87 * (double)rounds(256, 256));
+  struct {
+    PrefillNarrow shape;
+    double cost;
+  } const shapes[] = {{{64, 32}, 0.165}, {{64, 64}, 0.26}, {{96, 32}, 0.22}, {{96, 64}, 0.31}};
+  PrefillNarrow best{0, 0};
+  double least = 0.95 * wide;
+  for (const auto &s : shapes) {
+    const double cost = steps * s.cost * (double)rounds(s.shape.rows, s.shape.columns);
+    if (cost < least) least = cost, best = s.shape;
+  }
+  return best;
+}
 // The stream schedule of a whole-K dispatch of 256-row tiles, row_blocks x column_groups of them, K / 64 steps each,
 // in one dispatch. Whole rounds of kPrefillUnits tiles run as whole tiles (dp_tiles: whole column groups, so that the
 // row blocks divide the units), one a workgroup; the rest (stream_tiles, between half a round and a round and a
@@ -1005,6 +1030,9 @@ hipError_t launch_prefill_prepare(const uint16_t *input, uint32_t rows, uint32_t
 }
 
 hipError_t launch_prefill(uint32_t fmt, uint32_t epilogue, const PrefillArgs &a, hipStream_t stream) {
+  const uint32_t width = a.out_stride / 64;
+  const PrefillNarrow narrow = prefill_narrow(a.rows, width, a.K, prefill_split(a.rows, width, a.K));
+  if (narrow.rows) return launch_prefill_narrow(fmt, epilogue, a, narrow, stream);
   switch (fmt) {
     case SQ_FMT_AF4G32: return launch_format<SQ_FMT_AF4G32>(epilogue, a, stream);
     case SQ_FMT_AF4G64: return launch_format<SQ_FMT_AF4G64>(epilogue, a, stream);

@@ -66,6 +66,45 @@ def test_prefill_dense(fmt, rows):
     no_worse_than_staged(None, x, w, stats, f"prefill fmt {fmt} rows {rows}")
 
 
+@pytest.mark.parametrize("fmt", [oracle.FMT_AF4G64, oracle.FMT_Q4K, oracle.FMT_AF4G128, oracle.FMT_AF4G32] + NEW_FORMATS)
+@pytest.mark.parametrize("rows,n,k", [
+    (40, 1088, 768),      # 64 x 32: two or one steps a wave
+    (97, 2112, 1280),     # 64 x 32, a second row block of 33 rows, two or three steps a wave
+    (90, 5120, 512),      # 96 x 32, one step a wave
+    (128, 5120, 256),     # 64 x 64, half of the waves without steps
+    (200, 5120, 768),     # 96 x 64, the last row block of eight rows
+    (128, 27648, 512),    # 108 column groups: the wide tile of 128 rows
+])
+def test_prefill_tile_choice(fmt, rows, n, k):
+    """The narrow tile's shapes and the wide tile beside them, at row and K remainders, against the fp64 interval."""
+    rng = np.random.default_rng(rows + n + fmt)
+    w = make_weights(rng, fmt, n, k)
+    x = dense_inputs(rng, rows, k)
+    pick = np.unique(np.r_[np.arange(0, rows, 11), rows - 1])
+    check_projection(run_prefill([w], x)[pick], x[pick], w, f"tile choice fmt {fmt}, {rows} rows of {k} x {n}")
+
+
+@pytest.mark.parametrize("k", [64, 448])
+def test_prefill_narrow_epilogues_and_segments(k):
+    """The narrow tile under both epilogues and over a fused projection's segments, at K of one step and of seven."""
+    rng = np.random.default_rng(450 + k)
+    rows = 70
+    parts = [make_weights(rng, oracle.FMT_AF4G64, n, k) for n in (192, 64, 128)]
+    x = dense_inputs(rng, rows, k)
+    check_projection(run_prefill(parts, x), x, parts, "narrow segments")
+    w = parts[0]
+    plain = run_prefill([w], x)
+    residual = synthetic.bf16_bits(rng.uniform(-64, 64, (rows, w.n)).astype(np.float32))
+    check_projection(run_prefill([w], x, sq.EPILOGUE_RESIDUAL, residual=residual), x, w, "narrow residual",
+                     residual=residual)
+    gate = synthetic.bf16_bits(rng.uniform(-4, 4, (rows, w.n)).astype(np.float32))
+    got = synthetic.bf16_to_f32(run_prefill([w], x, sq.EPILOGUE_UP_WITH_GATE, gate_scratch=gate)).astype(np.float64)
+    gf = synthetic.bf16_to_f32(gate).astype(np.float64)
+    want = synthetic.bf16_to_f32(plain).astype(np.float64) * gf / (1 + np.exp(-gf))
+    ulp = np.ldexp(1.0, np.floor(np.log2(np.maximum(np.abs(want), 1e-30))).astype(int) - 7)
+    assert np.all(np.abs(got - want) <= ulp + 1e-30)
+
+
 def test_prefill_sparse_inputs_past_half_range():
     rng = np.random.default_rng(3)
     n, k = 256, 2048
