@@ -195,13 +195,16 @@ struct MoeExpertArgs {
   uint16_t *output;             // [tiles * tile_rows][output_size]
   const uint16_t *gate;         // a single tensor's up-with-gate operand (null otherwise)
   uint32_t K, output_size, tile_rows, max_tiles, fmt, gate_up, routes_per_row, experts, mode, gather;
-  uint32_t row_halves;          // 1: each tile's rows in 16-row halves, a workgroup each (tile_rows <= 32)
+  uint32_t single;              // 1: launch_moe_expert takes each tile alone, not with the expert's next
   uint32_t shared_fmt;          // the shared tiles' format (launch_moe_expert_small)
   uint32_t slices;              // set by launch_moe_expert_small: the K slices of a tile
+  uint32_t column_groups;       // set by launch_moe_expert: the workgroups of a tile
+  uint32_t listed;              // set by launch_moe_expert: its workgroups take their tiles from a sorted list
 };
+// Over 32-row tiles (moe_wide.hip).
 hipError_t launch_moe_expert(const MoeExpertArgs &args, hipStream_t stream);
 // The same pass over tiles of at most 16 rows (tile_rows) with K in slices: one launch for the routed tiles, in fmt,
-// and the shared ones, in shared_fmt (`mode` and `row_halves` are not read). Gate and up share each a format.
+// and the shared ones, in shared_fmt (`mode` and `single` are not read). Gate and up share each a format.
 hipError_t launch_moe_expert_small(const MoeExpertArgs &args, hipStream_t stream);
 hipError_t launch_moe_combine(const uint16_t *expert_output, const uint32_t *route_rows,
                               const float *routing_weights, const uint16_t *residual, uint16_t *output,

@@ -2,11 +2,10 @@
 // (gate and up in one pass, then down) and the combine (reference: kernels/shared/moe.metal:23-162,175-331,480-505
 // and kernels/shared/moe_gguf.metal:21-206).
 //
-// CDNA4 mapping. Each expert pass is the decode row tile's exact-operand inner loop (rowtile.hpp) per expert tile:
-// a wave streams one 64-column plane tile of its expert over all of K against the tile's (at most 32) grouped
-// rows; an expert's other tiles read the same weights while they are still in L2. The passes read their input rows
-// in the tile's read order (one 16-byte load per row block and group): the routed work opens by writing the block's
-// input rows in that order, and the gate/up pass writes the intermediate rows in it.
+// CDNA4 mapping. Each expert pass is the decode row tile's exact-operand arithmetic (rowtile.hpp) per expert tile: the
+// 8-row tiles here, the 32-row ones in moe_wide.hip. The passes read their input rows in the tile's read order (one
+// 16-byte chunk holds an MFMA operand): the routed work opens by writing the block's input rows in that order, and the
+// gate/up pass writes the intermediate rows in it.
 #include "kernels.hpp"
 #include "rowtile.hpp"
 
@@ -319,165 +318,6 @@ __global__ __launch_bounds__(512) void group_kernel(const uint32_t *selected, Sq
   }
 }
 
-// Workgroup (four 64-column tiles, expert tile): wave w streams column tile 4 blockIdx.x + w of the tile's expert
-// over all of K against the tile's rows (at most 32: the expert's grouped rows from tile * tile_rows), so each
-// wave owns its outputs and no wave waits on another. The gate/up pass reads its rows through the grouped routes
-// (row r of the tile is input row routes[r] / top_k: the reference's gather copy folds into these loads) and
-// writes bf16(bf16(up) silu(bf16(gate))); a gate and up of different formats run as two such gathering passes, the
-// gate's output feeding the up pass's epilogue; the down pass reads the grouped intermediate rows
-// (moe_gguf.metal:121-206, moe_expert_slab.h:13-99).
-// The passes that stream chunks of two groups with operands built just before their MFMAs: those of 4-bit affine
-// codes in groups of 32 or 64 (a gate/up pair then fits two waves a SIMD, a single tensor three), every
-// single-tensor pass whose scale groups fit a two-group chunk (the K-quants and 8-bit codes then fit two waves a SIMD
-// instead of one), and the Q4_K and Q5_K gate/up pairs, whose coefficients each lane derives for its own column only
-// (rowtile.hpp: 239 and 250 registers, two waves a SIMD). The other gate/up pairs (Q6_K's halves, 8-bit codes, groups
-// of 128) would spill there and keep four-group chunks with operands a group ahead, one wave a SIMD. Chunks hold
-// whole scale groups either way, so the sums are the same bits.
-template <uint32_t FMT>
-constexpr bool affine4_short() { return FMT == SQ_FMT_AF4G32 || FMT == SQ_FMT_AF4G64; }
-template <uint32_t FMT, int NT>
-constexpr bool short_chunks() {
-  return affine4_short<FMT>() || (NT == 1 && Fmt<FMT>::SG <= 2) || FMT == SQ_FMT_Q4K || FMT == SQ_FMT_Q5K;
-}
-template <uint32_t FMT, int NT>
-constexpr int expert_waves() { return affine4_short<FMT>() ? (NT == 2 ? 2 : 3) : short_chunks<FMT, NT>() ? 2 : 1; }
-
-// Rows row0..row0 + rows - 1 of tile `tile` (all of them, or a 16-row half of it).
-template <uint32_t FMT, int MB, int NT>
-__device__ __forceinline__ void expert_tile(const MoeExpertArgs &a, SqMoeTileDescriptor d, uint32_t tile,
-                                            uint32_t ct, uint32_t row0, uint32_t rows) {
-  using F = Fmt<FMT>;
-  const uint32_t column_tiles = a.output_size / 64;
-  const uint32_t first_row = tile * a.tile_rows + row0;
-  const int lane = threadIdx.x & 63, j = lane & 15, q = lane >> 4;
-  const uint32_t G = a.K >> 5;
-  // The plane tile: routed expert e's from tile slots[e] of its projection on, shared slice s's from tile s of the
-  // shared segment on.
-  const bool shared = d.expert >= a.experts;
-  // A down pass of two tensor slots (pair) streams column tiles ct and ct + 1 of its one tensor, both against the
-  // same input loads.
-  const bool pair = NT == 2 && !a.gate_up;
-  const uint32_t ptile = (shared ? d.expert - a.experts : a.slots[d.expert]) * column_tiles + ct;
-  const uint8_t *plane[NT], *high[NT], *meta[NT];
-#pragma unroll
-  for (int n = 0; n < NT; ++n) {
-    const int slot = pair ? 0 : n;
-    const size_t pt = ptile + (pair ? n : 0);
-    plane[n] = (shared ? a.shared_plane0[slot] : a.plane0[slot]) + (pt * G * 64 + lane) * F::P0;
-    high[n] = F::P1 ? (shared ? a.shared_plane1[slot] : a.plane1[slot]) + (pt * G * 64 + lane) * F::P1 : nullptr;
-    meta[n] = (shared ? a.shared_meta[slot] : a.meta[slot]) + (pt * (G / F::UNIT) * 64 + lane) * F::META;
-  }
-  // Lane (j, q) of row block b reads row 16 b + j (row 0 past the tile's rows: nothing stores those results), its
-  // 16-byte chunk q of each group in the read order.
-  const uint16_t *xrow[MB];
-#pragma unroll
-  for (int b = 0; b < MB; ++b) {
-    const uint32_t r = 16u * b + j < rows ? 16u * b + j : 0u;
-    const uint32_t source = a.gather ? a.routes[first_row + r] / a.routes_per_row : first_row + r;
-    xrow[b] = a.input + (size_t)source * a.K + 8 * q;
-  }
-  float acc[NT][4][MB][4];
-  clear(acc);
-  // Two register sets (one chunk of loads ahead): the passes are bound by instruction issue, and a third set for a
-  // gate/up pair only moves more of its MFMA results through the accumulation registers. Short chunks fit more
-  // waves a SIMD (expert_kernel), and each resident wave covers more of the others' dependency stalls.
-  constexpr bool kShort = short_chunks<FMT, NT>();
-  row_stream<FMT, MB, NT, 2, kShort ? 2 : 4, !kShort>(plane, high, meta, xrow, 0, G, acc);
-  // Column 16 t + j of the tile: the gathering passes store it at its place in the read order (chunk 4 g + j / 4 of
-  // group g = 2 ct + t / 2, then position 4 (t % 2) + j % 4), for the down pass; the down pass in column order.
-  const uint32_t column = a.gather ? 8 * (j >> 2) + (j & 3) : j;
-#pragma unroll
-  for (int t = 0; t < 4; ++t)
-#pragma unroll
-    for (int b = 0; b < MB; ++b)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const uint32_t r = 16u * b + 4u * q + i;
-        if (r >= rows) continue;
-        const uint32_t c = a.gather ? 32 * (t >> 1) + 4 * (t & 1) + column : 16 * t + column;
-        const size_t at = (size_t)(first_row + r) * a.output_size + ct * 64 + c;
-        if (pair) {
-          a.output[at] = f32_to_bf16(acc[0][t][b][i]);
-          a.output[at + 64] = f32_to_bf16(acc[NT - 1][t][b][i]);
-        } else if constexpr (NT == 2) {
-          const float g = bf16_to_f32(f32_to_bf16(acc[0][t][b][i])), u = bf16_to_f32(f32_to_bf16(acc[1][t][b][i]));
-          a.output[at] = f32_to_bf16(u * silu(g));
-        } else if (a.gate) {
-          const float u = bf16_to_f32(f32_to_bf16(acc[0][t][b][i]));
-          a.output[at] = f32_to_bf16(u * silu(bf16_to_f32(a.gate[at])));
-        } else {
-          a.output[at] = f32_to_bf16(acc[0][t][b][i]);
-        }
-      }
-}
-
-// The tile workgroup row y runs, longest first: the tiles of more than 16 rows (two row blocks, about twice the work)
-// in tile order, then the others in tile order, so that the cheap tiles fill the compute units' last round instead of
-// a few expensive ones trailing it. The workgroup ranks the live tiles itself (each thread counts a run of them, then
-// a scan of the counts); past kOrderedTiles live tiles it keeps the tile order.
-constexpr uint32_t kOrderedTiles = 2048;
-__device__ uint32_t longest_first_tile(const SqMoeTileDescriptor *tiles, uint32_t n, uint32_t y) {
-  constexpr uint32_t kThreads = 256, kWaves = kThreads / 64;
-  __shared__ uint32_t wave_total[kWaves], picked;
-  if (n > kOrderedTiles) return y;
-  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const uint32_t run = (n + kThreads - 1) / kThreads, begin = min(n, tid * run), end = min(n, begin + run);
-  uint32_t big = 0;
-  for (uint32_t t = begin; t < end; ++t) big += tiles[t].rows > 16;
-  // Inclusive scan of the threads' counts of big tiles.
-  uint32_t inclusive = big;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const uint32_t up = (uint32_t)__shfl_up((int)inclusive, d);
-    if (lane >= (uint32_t)d) inclusive += up;
-  }
-  if (lane == 63) wave_total[wave] = inclusive;
-  __syncthreads();
-  uint32_t before = 0, all = 0;
-#pragma unroll
-  for (uint32_t w = 0; w < kWaves; ++w) {
-    before += w < wave ? wave_total[w] : 0u;
-    all += wave_total[w];
-  }
-  const uint32_t big_before = before + inclusive - big;   // big tiles before this thread's run
-  // Row y takes big tile y (y < all), else small tile y - all; the thread whose run holds it writes its index.
-  const bool want_big = y < all;
-  const uint32_t rank = want_big ? y : y - all;
-  const uint32_t mine_before = want_big ? big_before : begin - big_before, mine = want_big ? big : end - begin - big;
-  if (rank >= mine_before && rank < mine_before + mine) {
-    uint32_t seen = mine_before;
-    for (uint32_t t = begin; t < end; ++t)
-      if ((tiles[t].rows > 16) == want_big && seen++ == rank) {
-        picked = t;
-        break;
-      }
-  }
-  __syncthreads();
-  return picked;
-}
-
-// Tiles of at most 16 rows (most of an expert's last tiles) take the one-block path. With row_halves the grid's x
-// holds two copies of the column groups, and copy h takes rows 16 h..16 h + 15 of each tile on the one-block path
-// (a launch of few tiles then fills twice the SIMDs; each row computes what it does in the whole tile).
-template <uint32_t FMT, int MB, int NT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(expert_waves<FMT, NT>())))
-void expert_kernel(MoeExpertArgs a) {
-  const uint32_t n = a.tile_count->tiles;
-  if (blockIdx.y >= n) return;
-  const uint32_t tile = longest_first_tile(a.tiles, n, blockIdx.y);
-  const uint32_t groups = a.row_halves ? gridDim.x / 2 : gridDim.x, half = blockIdx.x / groups;
-  const uint32_t ct = (blockIdx.x % groups * 4 + (threadIdx.x >> 6)) * (NT == 2 && !a.gate_up ? 2 : 1);
-  if (ct >= a.output_size / 64) return;
-  const SqMoeTileDescriptor d = a.tiles[tile];
-  if (a.mode != 2 && (d.expert >= a.experts) != (a.mode == 1)) return;
-  if (a.row_halves) {
-    if (16 * half < d.rows) expert_tile<FMT, 1, NT>(a, d, tile, ct, 16 * half, min(16u, d.rows - 16 * half));
-    return;
-  }
-  if (MB == 1 || d.rows <= 16) expert_tile<FMT, 1, NT>(a, d, tile, ct, 0, d.rows);
-  else expert_tile<FMT, MB, NT>(a, d, tile, ct, 0, d.rows);
-}
-
 // Wave `slice`'s groups of tensor slot n of column tile ct against the at most 16 rows of a small tile, into acc.
 template <uint32_t FMT>
 __device__ __forceinline__ void small_walk(const MoeExpertArgs &a, SqMoeTileDescriptor d, uint32_t first_row, int n,
@@ -496,7 +336,7 @@ __device__ __forceinline__ void small_walk(const MoeExpertArgs &a, SqMoeTileDesc
   const uint32_t r = (uint32_t)j < d.rows ? j : 0u;
   const uint32_t source = a.gather ? a.routes[first_row + r] / a.routes_per_row : first_row + r;
   const uint16_t *const xrow[1] = {a.input + (size_t)source * a.K + 8 * q};
-  row_stream<FMT, 1, 1, 2, F::P0 == 32 || F::P1 ? 2 : 4, false>(plane, high, meta, xrow, first, end, acc);
+  row_stream<FMT, 1, 1, 2, F::P0 == 32 || F::P1 ? 2 : 4>(plane, high, meta, xrow, first, end, acc);
 }
 
 // The expert passes of 8-row tiles (decode steps and the smallest chunks: an expert's one to eight rows). There are
@@ -539,7 +379,8 @@ void expert_small_kernel(MoeExpertArgs a) {
   for (uint32_t o = wave; o < per * 16; o += kSmallWaves) {
     const uint32_t c = o / 16, f = o % 16, ct = ct0 + c, r = 4u * q + (f & 3), t = f >> 2;
     if (ct >= column_tiles || r >= d.rows) continue;
-    // The gathering passes store in the read order, the down pass in column order (expert_tile).
+    // The gathering passes store at the column's place in the read order (chunk 4 g + j / 4 of its group, position
+    // 4 (t % 2) + j % 4), the down pass in column order.
     const uint32_t place = a.gather ? 32 * (t >> 1) + 4 * (t & 1) + 8 * (j >> 2) + (j & 3) : 16 * t + j;
     const size_t at = (size_t)(first_row + r) * a.output_size + ct * 64 + place;
     const uint32_t from = c * a.slices * tensors;
@@ -626,25 +467,6 @@ __global__ __launch_bounds__(256) void combine_kernel(const uint16_t *expert_out
   *(u32x4 *)(output + at) = out;
 }
 
-template <uint32_t FMT, int MB, int NT>
-hipError_t launch_expert_rows(const MoeExpertArgs &a, hipStream_t stream) {
-  const uint32_t per = NT == 2 && !a.gate_up ? 8 : 4;   // column tiles a workgroup
-  const dim3 grid((a.output_size / 64 + per - 1) / per * (a.row_halves ? 2 : 1), a.max_tiles), block(256);
-  hipLaunchKernelGGL((expert_kernel<FMT, MB, NT>), grid, block, 0, stream, a);
-  return hipGetLastError();
-}
-
-// The down pass over 4-bit affine codes in groups of 32 or 64 streams column tiles in pairs (an even count of them):
-// each input load then serves two tiles, for the same registers as a gate/up pair (two waves a SIMD instead of three;
-// the pass is bound by its vector memory instructions more than by its waves: c4 174 -> 168 us).
-template <uint32_t FMT>
-hipError_t launch_expert_format(const MoeExpertArgs &a, hipStream_t stream) {
-  const bool pairs = affine4_short<FMT>() && !a.gate_up && !a.gather && (a.output_size / 64) % 2 == 0;
-  if (a.row_halves)
-    return a.gate_up || pairs ? launch_expert_rows<FMT, 1, 2>(a, stream) : launch_expert_rows<FMT, 1, 1>(a, stream);
-  return a.gate_up || pairs ? launch_expert_rows<FMT, 2, 2>(a, stream) : launch_expert_rows<FMT, 2, 1>(a, stream);
-}
-
 }  // namespace
 
 hipError_t launch_moe_route_select(const float *scores, uint32_t stride, uint32_t *selected, float *weights,
@@ -683,21 +505,6 @@ hipError_t launch_moe_expert_small(const MoeExpertArgs &args, hipStream_t stream
   hipLaunchKernelGGL(expert_small_kernel, dim3((a.output_size / 64 + per - 1) / per, a.max_tiles),
                      dim3(64 * kSmallWaves), 0, stream, a);
   return hipGetLastError();
-}
-
-hipError_t launch_moe_expert(const MoeExpertArgs &a, hipStream_t stream) {
-  if (a.tile_rows != 32) return hipErrorInvalidValue;
-  switch (a.fmt) {
-    case SQ_FMT_AF4G32: return launch_expert_format<SQ_FMT_AF4G32>(a, stream);
-    case SQ_FMT_AF4G64: return launch_expert_format<SQ_FMT_AF4G64>(a, stream);
-    case SQ_FMT_AF4G128: return launch_expert_format<SQ_FMT_AF4G128>(a, stream);
-    case SQ_FMT_Q4K: return launch_expert_format<SQ_FMT_Q4K>(a, stream);
-    case SQ_FMT_Q5K: return launch_expert_format<SQ_FMT_Q5K>(a, stream);
-    case SQ_FMT_Q6K: return launch_expert_format<SQ_FMT_Q6K>(a, stream);
-    case SQ_FMT_Q80: return launch_expert_format<SQ_FMT_Q80>(a, stream);
-    case SQ_FMT_AF8G64: return launch_expert_format<SQ_FMT_AF8G64>(a, stream);
-    default: return hipErrorInvalidValue;
-  }
 }
 
 hipError_t launch_moe_combine(const uint16_t *expert_output, const uint32_t *route_rows, const float *weights,

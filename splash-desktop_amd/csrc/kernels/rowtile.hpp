@@ -365,14 +365,13 @@ __device__ __forceinline__ void row_slice(const RowBuffers<FMT, NT, MB, TB> &src
 // Adds groups first .. end - 1 of NT tensors' plane tiles to acc, as row_slice does, in one continuous stream: chunks
 // of CH groups, each chunk's loads (clamped to the last group, so every chunk issues as many) issued SETS - 1 chunks
 // ahead into a ring of SETS register sets; first is a multiple of CH and of the meta unit or lies CH-aligned inside a
-// longer one; AHEAD builds each group's operands a group ahead (else just before its
-// MFMAs). plane[n] and high[n] point at group 0 for the lane, meta[n] at unit 0 of the lane's own column l (one
+// longer one. plane[n] and high[n] point at group 0 for the lane, meta[n] at unit 0 of the lane's own column l (one
 // load per unit and tensor, spread_coefs hands each lane the columns its MFMA blocks hold). The input rows come in the
 // tile's read order
 // (16-byte chunk 4 g + c of a row: inputs 32 g + 4 c .. +3 then 32 g + 16 + 4 c .. +3), so each group of a row block
 // is one 16-byte load a lane, half the vector memory instructions of two 8-byte loads from a row in input order:
 // xrow[b] points at chunk q of group 0 of the lane's row 16 b + j.
-template <uint32_t FMT, int MB, int NT, int SETS = 2, int CH = 4, bool AHEAD = true>
+template <uint32_t FMT, int MB, int NT, int SETS = 2, int CH = 4>
 __device__ __forceinline__ void row_stream(const uint8_t *const (&plane)[NT], const uint8_t *const (&high)[NT],
                                            const uint8_t *const (&meta)[NT], const uint16_t *const (&xrow)[MB],
                                            uint32_t first, uint32_t end, float (&acc)[NT][4][MB][4]) {
@@ -402,32 +401,19 @@ __device__ __forceinline__ void row_stream(const uint8_t *const (&plane)[NT], co
     }
   };
   f32x4 C[NT][4][MB], C2[NT][4][MB], S[MB], S2[MB];
-  // Each group's exact operands are built one group ahead, into the other of two operand sets, so that building
-  // them interleaves with the previous group's MFMAs; 8-bit codes (two operand sets a group), and callers that ask
-  // for it to fit the registers, build them just before their MFMAs.
-  constexpr bool kAhead = F::P0 != 32 && AHEAD;
-  u32x4 lo[2][NT][4], hi[2][NT][4];
-  const auto prepare = [&](int set, int u, int os) __attribute__((always_inline)) {
-#pragma unroll
-    for (int n = 0; n < NT; ++n) row_operands<FMT>(codes[set][n][u], hshift, cc, lo[os][n], hi[os][n]);
-  };
+  u32x4 lo[NT][4], hi[NT][4];
   const int j = threadIdx.x & 15;
-  const auto compute = [&](uint32_t c, int set, int next_set) __attribute__((always_inline)) {
+  const auto compute = [&](uint32_t c, int set) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < CH; ++u) {
       const uint32_t g = first + c * CH + u;
-      const int os = kAhead ? u & 1 : 0;   // CH is even: group g's operands sit in set u % 2
       if (g < end) {
         u32x4 x[MB];
 #pragma unroll
         for (int b = 0; b < MB; ++b) x[b] = xv[set][b][u];
-        if constexpr (!kAhead) prepare(set, u, 0);
-        row_group_mfma<FMT, MB, NT>(x, lo[os], hi[os], u % SG == 0, C, C2, S, S2);
-        // The next group's operands (the last group of a chunk takes the next chunk's first).
-        if constexpr (kAhead) {
-          if (u + 1 < CH) prepare(set, u + 1, os ^ 1);
-          else prepare(next_set, 0, os ^ 1);
-        }
+#pragma unroll
+        for (int n = 0; n < NT; ++n) row_operands<FMT>(codes[set][n][u], hshift, cc, lo[n], hi[n]);
+        row_group_mfma<FMT, MB, NT>(x, lo, hi, u % SG == 0, C, C2, S, S2);
         if ((u + 1) % SG == 0) {
           MetaWords unit[NT];
 #pragma unroll
@@ -442,13 +428,12 @@ __device__ __forceinline__ void row_stream(const uint8_t *const (&plane)[NT], co
   };
 #pragma unroll
   for (int c = 0; c < SETS - 1; ++c) issue(c, c);
-  if constexpr (kAhead) prepare(0, 0, 0);
   for (uint32_t c = 0; c < chunks; c += SETS) {
 #pragma unroll
     for (int k = 0; k < SETS; ++k) {
       issue(c + k + SETS - 1, (k + SETS - 1) % SETS);
       __builtin_amdgcn_sched_barrier(0);
-      compute(c + k, k, (k + 1) % SETS);
+      compute(c + k, k);
     }
   }
 }

@@ -246,6 +246,24 @@ def test_moe_small_tile_slices(fmt, hidden, inner):
     check_block(block, x, scores, 3, residual, "decode")
 
 
+@pytest.mark.parametrize("fmt", [oracle.FMT_AF4G32, oracle.FMT_AF4G64, oracle.FMT_AF4G128, oracle.FMT_AF8G64,
+                                 oracle.FMT_Q4K, oracle.FMT_Q5K, oracle.FMT_Q6K, oracle.FMT_Q80])
+@pytest.mark.parametrize("rows,hidden,inner", [
+    (150, 1024, 256),    # gate/up from the sorted work list, down by tile; experts of one to four tiles
+    (75, 256, 1280),   # gate/up by tile, down from the list; column groups short of a workgroup's
+])
+def test_moe_tile_pairs(fmt, rows, hidden, inner):
+    """32-row tiles two of an expert at a time: experts of odd and even tile counts, short last tiles, both ways a
+    launch's workgroups find their tiles, with a shared slice of another format beside (each tile of it alone)."""
+    rng = np.random.default_rng(rows + fmt)
+    block = Block(rng, 6, hidden, inner, fmt=fmt, shared=1, gated=True, shared_fmt=oracle.FMT_Q80
+                  if fmt != oracle.FMT_Q80 else oracle.FMT_AF4G64)
+    x = synthetic.activations(rng, rows, hidden)
+    scores = synthetic.router_logits(rng, rows, 6)
+    scores[:, 0] += 3   # the first expert takes nearly every row
+    check_block(block, x, scores, 2, None)
+
+
 @pytest.mark.parametrize("rows,phase", [(48, "prefill"), (5, "decode")])
 def test_moe_projections_in_formats_of_their_own(rows, phase):
     """Every projection in its own format (MoE.cpp:27-62): a routed gate and up of different formats (a gate pass and
