@@ -22,6 +22,16 @@ namespace {
 // The most waves a row-tile workgroup holds, so that a wave's registers fit without spilling: 16 (128 registers) for
 // one tensor of 16 rows, 4 (512) for a gate/up pair of 32 rows, else 8 (256).
 constexpr uint32_t row_max_waves(int mb, int nt) { return mb == 1 && nt == 1 ? 16 : mb == 2 && nt == 2 ? 4 : 8; }
+// Slices of kWideGroups groups (32 rows of one tensor in a format of kWideFormat) run in kWideWaves waves, one a SIMD
+// (decode_layout).
+constexpr uint32_t kWideGroups = 40, kWideWaves = 4;
+template <uint32_t FMT>
+constexpr bool kWideFormat = Fmt<FMT>::P1 == 0;
+template <>
+inline constexpr bool kWideFormat<kSegmentFormats> = false;
+constexpr uint32_t row_slots(int mb, int gw, int nt) {
+  return gw == (int)kWideGroups ? kWideWaves : row_max_waves(mb, nt);
+}
 
 // Wave `slice`'s K slice (groups gb.. of which `live` are in the slice) of plane tile `tile` of segment `seg`, in
 // format FMT, into acc. TB 1: column block cs of the tile only, lane (j, q) loading chunk q of column 16 cs + j and
@@ -76,7 +86,7 @@ __global__ __launch_bounds__(64 * row_max_waves(MB, NT)) void row_kernel(DecodeA
   // The slices' reduction buffer; during the walk each wave's own part of it (A floats a lane, at least MB KiB) is
   // its activations' LDS slot, which the wave leaves before writing its sums there.
   constexpr uint32_t FO = TB * MB * 4;   // outputs per tensor
-  __shared__ float red[row_max_waves(MB, NT) * A * 64];
+  __shared__ float red[row_slots(MB, GW, NT) * A * 64];
   static_assert(A * 64 * 4 >= MB * 1024, "a wave's reduction slot holds its activations' slot");
   uint8_t *const xlds = (uint8_t *)(red + slice * A * 64);
   if constexpr (FMT == kSegmentFormats)
@@ -128,7 +138,7 @@ __global__ __launch_bounds__(64 * row_max_waves(MB, NT)) void row_kernel(DecodeA
     for (int n = 0; n < NT; ++n) {
       // Every wave slot's read goes out at once (slots past the workgroup's waves hold nothing the sum takes), then
       // the adds run in slice order.
-      constexpr uint32_t kSlots = row_max_waves(MB, NT);
+      constexpr uint32_t kSlots = row_slots(MB, GW, NT);
       float part[kSlots], sum = 0.0f;
 #pragma unroll
       for (uint32_t w = 0; w < kSlots; ++w) part[w] = red[(w * A + n * FO + f) * 64 + lane];
@@ -204,6 +214,13 @@ hipError_t launch_mb(const DecodeArgs &a, uint32_t tiles, DecodeLayout layout, h
   switch (layout.ks) {
     case 8: launch_gw<FMT, MB, 8, NT, EP, F32OUT>(a, tiles, layout, stream); break;
     case 16: launch_gw<FMT, MB, 16, NT, EP, F32OUT>(a, tiles, layout, stream); break;
+    case kWideGroups:
+      if constexpr (NT == 1 && MB == 2 && kWideFormat<FMT>) {
+        hipLaunchKernelGGL((row_kernel<FMT, MB, kWideGroups, NT, EP, F32OUT, 4>), dim3(tiles, a.splits),
+                           dim3(64 * layout.nb), 0, stream, a);
+        break;
+      }
+      return hipErrorInvalidValue;
     default:
       if constexpr (NT == 1) launch_gw<FMT, MB, 32, NT, EP, F32OUT>(a, tiles, layout, stream);
       break;
@@ -247,6 +264,13 @@ DecodeLayout decode_layout(uint32_t fmt, uint32_t blocks, uint32_t K, uint32_t s
   const uint32_t gs = units / splits * sg;
   const uint32_t most = rows <= kColumnTileRows ? kColumnMaxWaves : row_max_waves(rows <= 16 ? 1 : 2, pair ? 2 : 1);
   const uint32_t tiles = blocks / 4;
+  // Past one round of workgroups, 32 rows of one tensor whose slices of 32 groups would be five waves take four of 40:
+  // the fifth wave doubles up on the first SIMD, and a second workgroup's would need four waves' registers there, so a
+  // compute unit held one workgroup where four waves leave room for two. Measured (M = 32, K 5120, N 17408 / 27648): Q4_K
+  // 41.1 / 41.4 -> 35.5 / 37.5 us, af4g64 36.8 / 37.9 -> 35.0 / 36.5, Q8_0 57.0 / 59.7 -> 50.4 / 53.8; with plane1 bits
+  // the longer slice spills (Q6_K 67.6 -> 138.6), so those formats and mixed segments keep 32.
+  if (rows > 16 && !pair && !sq_format(fmt).plane1_bytes && tiles * splits > kDecodeUnits && gs > 4 * kColumnMaxGroups && gs <= kWideWaves * kWideGroups)
+    return {kWideWaves, kWideGroups};
   if (rows > kColumnTileRows && !pair && sq_format(fmt).plane0_bytes == 16 && tiles * splits > kDecodeUnits &&
       (gs + kColumnMaxGroups - 1) / kColumnMaxGroups <= most)
     return {(gs + kColumnMaxGroups - 1) / kColumnMaxGroups, kColumnMaxGroups};
@@ -271,8 +295,9 @@ hipError_t launch_decode(uint32_t fmt, uint32_t epilogue, bool f32_output, const
   uint32_t tiles = 0;
   for (uint32_t s = 0; s < args.segments; ++s) tiles += args.seg[s].tiles;
   const bool pair = args.gate.plane0 != nullptr;
-  const DecodeLayout layout = decode_layout(layout_format(fmt, args), tiles * 4, args.K, args.splits, pair, args.rows);
+  DecodeLayout layout = decode_layout(layout_format(fmt, args), tiles * 4, args.K, args.splits, pair, args.rows);
   if (!layout.nb) return hipErrorInvalidValue;
+  if (fmt == kSegmentFormats && layout.ks == kWideGroups) layout = {5, kColumnMaxGroups};   // the same groups
   switch (fmt) {
     case SQ_FMT_AF4G32: return launch_format<SQ_FMT_AF4G32>(epilogue, f32_output, pair, args, tiles, layout, stream);
     case SQ_FMT_AF4G64: return launch_format<SQ_FMT_AF4G64>(epilogue, f32_output, pair, args, tiles, layout, stream);

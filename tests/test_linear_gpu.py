@@ -470,6 +470,25 @@ def test_row_tile_long_slices(fmt, rows, k):
     assert stats["rel_l2"] <= ref_l2 * 1.10 + 1e-6
 
 
+@pytest.mark.parametrize("fmt,rows,k", [(oracle.FMT_AF4G32, 17, 4352), (oracle.FMT_AF4G64, 32, 5120),
+                                        (oracle.FMT_AF4G128, 20, 4608), (oracle.FMT_Q4K, 32, 5120),
+                                        (oracle.FMT_Q4K, 31, 4352), (oracle.FMT_Q5K, 24, 4864),
+                                        (oracle.FMT_Q80, 24, 4352), (oracle.FMT_AF8G64, 32, 5120)])
+def test_row_tile_slices_of_forty_groups(fmt, rows, k):
+    """17 to 32 rows past one round of workgroups (257 tiles): formats without plane1 bits run 129 to 160 groups as four
+    slices of 40, the last of 16 (K 4352) to 40 (K 5120) groups; Q5_K keeps slices of 32. Every
+    output against fp64 with the register tile's bound, and the last row's bits the same in 17 rows."""
+    n = 64 * 257
+    w = shape_weights(fmt, n, k, 23 + fmt)
+    rng = np.random.default_rng(500 + rows + fmt + k)
+    x = dense_inputs(rng, rows, k)
+    proj = sq.projection(w.segment())
+    got = run_plan(staged(n, k, rows, 1), proj, x, n)
+    check_decode(got, x, w, f"fmt {fmt} {n}x{k} rows {rows}")
+    again = run_plan(staged(n, k, 17, 1), proj, x[-17:], n)
+    assert np.array_equal(again[-1], got[-1])
+
+
 NEW_FORMATS = [oracle.FMT_Q5K, oracle.FMT_Q6K, oracle.FMT_Q80, oracle.FMT_AF8G64]
 
 
