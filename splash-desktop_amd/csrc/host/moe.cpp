@@ -250,6 +250,7 @@ void MoE::addRouted(hipStream_t graph, const MoeBuffers &b, const MoeWeights &w,
   a.routes = sc.groupedRoutes.as<const uint32_t>();
   a.routes_per_row = s.routesPerToken();
   a.experts = s.experts;
+  a.routed = plan.rows() * s.expertsPerToken;
   // Plane views of tensor slot n: the routed projection's and the shared one's.
   const auto bind = [&](int n, const QuantizedSegment &routed, const QuantizedSegment &shared) {
     a.plane0[n] = routed.plane0.as<const uint8_t>();

@@ -195,6 +195,7 @@ struct MoeExpertArgs {
   uint16_t *output;             // [tiles * tile_rows][output_size]
   const uint16_t *gate;         // a single tensor's up-with-gate operand (null otherwise)
   uint32_t K, output_size, tile_rows, max_tiles, fmt, gate_up, routes_per_row, experts, mode, gather;
+  uint32_t routed;              // the routed routes of the block (rows x experts a row)
   uint32_t single;              // 1: launch_moe_expert takes each tile alone, not with the expert's next
   uint32_t shared_fmt;          // the shared tiles' format (launch_moe_expert_small)
   uint32_t slices;              // set by launch_moe_expert_small: the K slices of a tile

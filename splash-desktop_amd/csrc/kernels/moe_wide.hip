@@ -8,8 +8,8 @@
 // of both tensors' 32 columns, two a SIMD, took 206 us where this takes 160: Q4_K gate/up of 1999 rows of 8 routes over
 // 256 experts of 2048 x 512; the row tile's 16x16x32 walk of 32 rows, 213; VALU issue 55% of the dispatch). Per step of 64 inputs
 //  - the workgroup's rows come 128 bytes a row (eight lanes a row, whole cache lines) through registers into LDS, one
-//    step ahead, in two stages with one barrier a step, with each group's input sums (four lanes a group) beside them;
-//    every wave reads its MFMA fragments from there;
+//    step ahead (32 rows and fewer: two), in two stages with one barrier each, with each group's input sums (four lanes a
+//    group) beside them; every wave reads its MFMA fragments from there;
 //  - a lane holds one column's codes of one of the step's groups (lane l: column l % 32, group l / 32), so two
 //    v_permlane32_swap turn a block's words into both groups' B operands, the lane derives one (column, group)'s
 //    coefficients, one more swap gives every lane its column's scales of both groups, and the offsets already lie in the
@@ -17,6 +17,8 @@
 //  - each scale group closes as acc += s * sum x (128 + q) on the VALU, and the offsets of both groups, (z - 128 s) *
 //    sum x, in one 32x32x2 fp32 MFMA a row block.
 // The passes are bound by instruction issue; a row's result depends only on its own activations.
+#include <type_traits>
+
 #include "kernels.hpp"
 #include "rowtile.hpp"
 
@@ -68,16 +70,36 @@ __device__ __forceinline__ float quad_total(float v) {
   return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xF, 0xF, false));
 }
 
-// The walk of one wave over RB blocks of 32 rows: acc[b] += its 32 columns' sums. plane, high and meta: the plane tile,
-// c0 the wave's first column of it; xrow: row 8 wave + lane / 8 (RB 1: 4 wave + lane / 8, lanes 0..31), chunk lane % 8.
-template <uint32_t FMT, int RB>
+// The row of the workgroup's whose chunk lane % 8 the lane stages.
+template <int RB>
+__device__ __forceinline__ uint32_t stage_row() {
+  return RB == 2 ? threadIdx.x >> 3 : 4 * (threadIdx.x >> 6) + ((threadIdx.x >> 3) & 3);
+}
+// That row in the input: a pointer to the lane's chunk, or, in the formats whose walk would spill the pointer (each reload
+// then waits for every load in flight), the 64-input span it begins at. Measured, block times at 33 / 128 rows of eight
+// routes over 256 experts of 2048 x 512, pointer -> span: af4g128 99 / 139 -> 89 / 130 us, Q6_K 143 / 199 -> 137 / 194;
+// af4g64 84 / 123 -> 86 / 127 (the span's address takes instructions), so the formats that don't spill keep the pointer.
+template <uint32_t FMT>
+constexpr bool kRowSpans = FMT == SQ_FMT_AF4G128 || FMT == SQ_FMT_Q6K;
+template <uint32_t FMT>
+using RowSource = std::conditional_t<kRowSpans<FMT>, uint32_t, const uint16_t *>;
+
+// The walk of one wave over RB blocks of 32 rows: acc[b] += its 32 columns' sums, in registers 0..LIVE - 1 (LIVE 8: rows
+// 0..15 of a block). plane, high and meta: the plane tile, c0 the wave's first column of it; row: the lane's row, of the
+// workgroup's `rows`. One block stages two steps at a time (lanes 0..31 the even step's rows, 32..63 the odd one's), in
+// four half stages: one barrier and one wait for rows every two steps. Tiles of few rows run as many steps as tall ones
+// and hold little to do in each, so they were bound by that wait: 64 rows of eight routes over 256 af4g64 experts of
+// 2048 x 512, a step at a time with every wave staging and sixteen registers closed, 143 us the block; so, 115.
+template <uint32_t FMT, int RB, int LIVE>
 __device__ __forceinline__ void wide_walk(const MoeExpertArgs &a, const uint8_t *plane, const uint8_t *high,
-                                          const uint8_t *meta, uint32_t c0, const uint16_t *xrow, uint8_t *lds,
-                                          f32x16 (&acc)[RB]) {
+                                          const uint8_t *meta, uint32_t c0, RowSource<FMT> row, uint32_t rows,
+                                          uint8_t *lds, f32x16 (&acc)[RB]) {
   using F = Fmt<FMT>;
   constexpr int SG = F::SG, NH = F::HALVES ? 2 : 1;
   const int lane = threadIdx.x & 63, l32 = lane & 31, h = lane >> 5;
-  const uint32_t wave = threadIdx.x >> 6, G = a.K >> 5, steps = G / 2;
+  constexpr uint32_t kSteps = RB == 2 ? 1 : 2;   // steps staged at a time
+  constexpr int kRows = RB * 32 * 128, kStage = kStageBytes / kSteps;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), G = a.K >> 5, steps = G / 2;
   const CodeConstants cc = make_code_constants();
 
   const uint32_t col = c0 + l32;
@@ -100,17 +122,23 @@ __device__ __forceinline__ void wide_walk(const MoeExpertArgs &a, const uint8_t 
   const auto load_meta_of = [&](uint32_t step) __attribute__((always_inline)) {
     return buffer_meta<FMT>(metas, mv, 2 * step / F::UNIT * 64 * F::META);
   };
+  // Waves whose rows all lie past the workgroup's stage none: what the stages hold there reaches only outputs that are
+  // not stored.
   u32x4 x;
-  const bool loads = RB == 2 || lane < 32;
+  const uint32_t my_row = stage_row<RB>();
+  const bool loads = RB == 2 || 4 * wave < rows;
   const auto load_rows = [&](uint32_t step) __attribute__((always_inline)) {
-    if (loads) x = *(const u32x4 *)(xrow + step * 64);
+    const uint32_t at = min(RB == 2 ? step : step + h, steps - 1);
+    if (!loads) return;
+    if constexpr (!kRowSpans<FMT>) x = *(const u32x4 *)(row + at * 64);
+    else if constexpr (RB == 2) x = ((const u32x4 *)a.input + 8 * at)[8 * (size_t)row + (lane & 7)];
+    else x = ((const u32x4 *)a.input)[8 * (size_t)(row + at) + (lane & 7)];
   };
-  const uint32_t my_row = (RB == 2 ? 8 : 4) * wave + (lane >> 3);
-  const auto store_rows = [&](uint32_t stage) __attribute__((always_inline)) {
-    uint8_t *const to = lds + stage * kStageBytes;
+  const auto store_rows = [&](uint32_t step) __attribute__((always_inline)) {
+    uint8_t *const to = lds + (RB == 2 ? step & 1 : (step & 2) + h) * kStage;
     if (loads) {
       *(u32x4 *)(to + stage_at(my_row, lane & 7)) = x;
-      float *const sums = (float *)(to + kRowBytes) + my_row * (2 * NH) + ((lane >> 2) & 1);
+      float *const sums = (float *)(to + kRows) + my_row * (2 * NH) + ((lane >> 2) & 1);
       const float first = quad_of(x[0], x[1]), second = quad_of(x[2], x[3]);
       if constexpr (F::HALVES) {
         const float s0 = quad_total(first), s1 = quad_total(second);
@@ -129,10 +157,14 @@ __device__ __forceinline__ void wide_walk(const MoeExpertArgs &a, const uint8_t 
 #pragma unroll
   for (int r = 0; r < 16; ++r) zero[r] = 0.0f;
   f32x16 C[RB];
+  const auto close = [&](f32x16 &to, float scale, const f32x16 &c) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < LIVE; ++r) to[r] = fmaf(scale, c[r], to[r]);
+  };
 
   const auto compute = [&](uint32_t step, const Words &w, const MetaWords &meta_words) __attribute__((always_inline)) {
-    const uint8_t *stage = lds + (step & 1) * kStageBytes;
-    const float *sums = (const float *)(stage + kRowBytes);
+    const uint8_t *stage = lds + (step & (2 * kSteps - 1)) * kStage;
+    const float *sums = (const float *)(stage + kRows);
     // The lane's coefficients (its column's in group 2 step + h).
     float s[2], zc[2];
     const uint32_t own = 2 * step + h;
@@ -210,9 +242,7 @@ __device__ __forceinline__ void wide_walk(const MoeExpertArgs &a, const uint8_t 
 #pragma unroll
           for (int b = 0; b < RB; ++b) C[b] = mfma32(half_of(xa[b], xb[b], m), half_of(lo[0], lo[1], m), zero);
 #pragma unroll
-          for (int b = 0; b < RB; ++b)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[b][r] = fmaf(sg[m], C[b][r], acc[b][r]);
+          for (int b = 0; b < RB; ++b) close(acc[b], sg[m], C[b]);
         }
       } else {
 #pragma unroll
@@ -227,9 +257,7 @@ __device__ __forceinline__ void wide_walk(const MoeExpertArgs &a, const uint8_t 
         }
         if (last)
 #pragma unroll
-          for (int b = 0; b < RB; ++b)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[b][r] = fmaf(sg[0], C[b][r], acc[b][r]);
+          for (int b = 0; b < RB; ++b) close(acc[b], sg[0], C[b]);
       }
     }
     // Both groups' offsets (a scale group over both or over several steps: its offset times each group's sum).
@@ -247,7 +275,7 @@ __device__ __forceinline__ void wide_walk(const MoeExpertArgs &a, const uint8_t 
   MetaWords m[kUnitMeta ? 2 : kRing];
   load_rows(0);
   store_rows(0);
-  load_rows(min(1u, steps - 1));   // before the codes, as in the loop, so that waiting for them does not wait for those
+  load_rows(kSteps);   // before the codes, as in the loop, so that waiting for them does not wait for those
 #pragma unroll
   for (int k = 0; k < kAhead; ++k) {
     load(min((uint32_t)k, steps - 1), w[k]);
@@ -255,9 +283,11 @@ __device__ __forceinline__ void wide_walk(const MoeExpertArgs &a, const uint8_t 
   }
   if constexpr (kUnitMeta) m[0] = load_meta_of(0);
   const auto run = [&](uint32_t at, int k) __attribute__((always_inline)) {
-    step_barrier();   // the stage's rows are in, and the other stage's reads are done
-    store_rows((at + 1) & 1);
-    load_rows(min(at + 2, steps - 1));
+    if (RB == 2 || k % 2 == 0) {
+      step_barrier();   // the stage's rows are in, and the other stage's reads are done
+      store_rows(at + kSteps);
+      load_rows(at + 2 * kSteps);
+    }
     load(min(at + kAhead, steps - 1), w[(k + kAhead) % kRing]);
     if constexpr (!kUnitMeta) m[(k + kAhead) % kRing] = load_meta_of(min(at + kAhead, steps - 1));
     compute(at, w[k], m[kUnitMeta ? 0 : k]);
@@ -383,10 +413,14 @@ __device__ uint32_t work_list(const MoeExpertArgs &a, uint32_t n, uint16_t *expe
 // A workgroup runs one column group of a tile and, if it is the expert's next, the tile after it (tiles pair from the
 // expert's first on). Over a long K it takes its tiles from the work list, the tall ones first: entries go round the
 // XCDs (workgroup b runs on XCD b % 8), an entry's column groups on one XCD, whose L2 they share its rows in. Over a
-// short K the list costs more than the order gains, and the workgroups go by tile, those of a pair's second tile
+// short K, or where the routed experts hold at most 24 rows on average (most are then one tile, and the order has nothing
+// to put first), the list costs more than the order gains, and the workgroups go by tile, those of a pair's second tile
 // returning at once; tiles go round the XCDs two by two, so that those do not idle the XCDs of one parity. Measured (35B
 // layer, 1999 rows), list against tiles: gate/up of K 2048 160 against 178 us, down of K 512 136 against 121; 512 rows,
-// down of K 768 45 against 50.
+// down of K 768 45 against 50. By rows an expert, af4g64 blocks, list against tiles: 4 (256 experts of 2048 x 512) 130
+// against 125 us, 17 (60 of 2048 x 1280) 103 against 100, 32 (128 of 2048 x 768) 157 against 167, 34 (60) 139 against 153.
+// Launches that hold shared tiles keep the list: Q8_0 with its shared slice, 64 rows, 198 against 219.
+constexpr uint32_t kListedRows = 24;
 template <uint32_t FMT>
 __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(4)))
 void expert_wide_kernel(MoeExpertArgs a) {
@@ -447,9 +481,11 @@ void expert_wide_kernel(MoeExpertArgs a) {
   const uint8_t *const high = F::P1 ? (shared ? a.shared_plane1[t] : a.plane1[t]) + pt * G * 64 * F::P1 : nullptr;
   const uint8_t *const meta = (shared ? a.shared_meta[t] : a.meta[t]) + pt * (G / F::UNIT) * 64 * F::META;
   const bool tall = rows > 32;
-  const uint32_t r = (tall ? 8 : 4) * wave + (lane >> 3), row = r < rows ? r : 0u;
+  const uint32_t r = tall ? stage_row<2>() : stage_row<1>(), row = r < rows ? r : 0u;
   const uint32_t source = a.gather ? a.routes[first_row + row] / a.routes_per_row : first_row + row;
-  const uint16_t *const xrow = a.input + (size_t)source * a.K + 8 * (lane & 7);
+  RowSource<FMT> from;
+  if constexpr (kRowSpans<FMT>) from = source * (a.K / 64);
+  else from = a.input + (size_t)source * a.K + 8 * (lane & 7);
   const auto clear16 = [&](f32x16 &v) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) v[i] = 0.0f;
@@ -458,12 +494,13 @@ void expert_wide_kernel(MoeExpertArgs a) {
     f32x16 acc[2];
     clear16(acc[0]);
     clear16(acc[1]);
-    wide_walk<FMT, 2>(a, plane, high, meta, 32 * (block & 1), xrow, lds, acc);
+    wide_walk<FMT, 2, 16>(a, plane, high, meta, 32 * (block & 1), from, rows, lds, acc);
     wide_store(a, acc, first_row, rows, 32 * c, live, lds);
   } else {
     f32x16 acc[1];
     clear16(acc[0]);
-    wide_walk<FMT, 1>(a, plane, high, meta, 32 * (block & 1), xrow, lds, acc);
+    if (rows > 16) wide_walk<FMT, 1, 16>(a, plane, high, meta, 32 * (block & 1), from, rows, lds, acc);
+    else wide_walk<FMT, 1, 8>(a, plane, high, meta, 32 * (block & 1), from, rows, lds, acc);
     wide_store(a, acc, first_row, rows, 32 * c, live, lds);
   }
 }
@@ -473,7 +510,7 @@ hipError_t launch_format(const MoeExpertArgs &args, hipStream_t stream) {
   MoeExpertArgs a = args;
   const uint32_t blocks = a.output_size / 32, per = a.gate_up ? kTensorWaves : kWaves;
   a.column_groups = (blocks + per - 1) / per;
-  a.listed = a.K >= 768;
+  a.listed = a.K >= 768 && (a.mode != 0 || a.routed > kListedRows * a.experts);
   const uint32_t grid = a.column_groups * ((a.max_tiles + 15) / 16) * 16;
   hipLaunchKernelGGL(expert_wide_kernel<FMT>, dim3(grid), dim3(64 * kWaves), 0, stream, a);
   return hipGetLastError();

@@ -264,6 +264,30 @@ def test_moe_tile_pairs(fmt, rows, hidden, inner):
     check_block(block, x, scores, 2, None)
 
 
+@pytest.mark.parametrize("fmt,inner", [(oracle.FMT_AF4G32, 64), (oracle.FMT_AF4G64, 320), (oracle.FMT_AF4G128, 384),
+                                       (oracle.FMT_AF8G64, 320), (oracle.FMT_Q80, 64), (oracle.FMT_Q4K, 256),
+                                       (oracle.FMT_Q5K, 512), (oracle.FMT_Q6K, 256)])
+def test_moe_rows_in_tiles_of_any_height(fmt, inner):
+    """A row's bits are the same whatever rows share its 32-row tile, one tile or two to a workgroup (tiles staged a
+    step or two at a time, with one or two wave-rows' worth of rows live, at odd counts of 64-input steps down to one),
+    and the same in 8-row tiles of any height; and each block within the bound of every block here."""
+    rng = np.random.default_rng(1700 + fmt)
+    block = Block(rng, 2, 1024, inner, fmt=fmt)
+    x = synthetic.activations(rng, 70, 1024)
+    scores = synthetic.router_logits(rng, 70, 2)
+    scores[:, 0] += 20   # every row to the first expert
+    _, tiles, whole = check_block(block, x, scores, 1, None)
+    assert list(tiles[:, 1]) == [32, 32, 6]
+    for rows in (3, 5, 8, 9, 16, 17, 32, 33, 41, 49, 64):
+        _, _, got = run_moe(block, x[:rows], scores[:rows], 1)
+        assert np.array_equal(got, whole[:rows]), rows
+    _, tiles, small = check_block(block, x[:31], scores[:31], 1, None, "decode")
+    assert list(tiles[:, 1]) == [8, 8, 8, 7]
+    for rows in (1, 7, 8, 20):
+        _, _, got = run_moe(block, x[:rows], scores[:rows], 1, phase="decode")
+        assert np.array_equal(got, small[:rows]), rows
+
+
 @pytest.mark.parametrize("rows,phase", [(48, "prefill"), (5, "decode")])
 def test_moe_projections_in_formats_of_their_own(rows, phase):
     """Every projection in its own format (MoE.cpp:27-62): a routed gate and up of different formats (a gate pass and
