@@ -336,7 +336,7 @@ __device__ __forceinline__ void small_walk(const MoeExpertArgs &a, SqMoeTileDesc
   const uint32_t r = (uint32_t)j < d.rows ? j : 0u;
   const uint32_t source = a.gather ? a.routes[first_row + r] / a.routes_per_row : first_row + r;
   const uint16_t *const xrow[1] = {a.input + (size_t)source * a.K + 8 * q};
-  row_stream<FMT, 1, 1, 2, F::P0 == 32 || F::P1 ? 2 : 4>(plane, high, meta, xrow, first, end, acc);
+  row_stream<FMT, 1, 1, 2, F::SG <= 2 ? 2 : 4>(plane, high, meta, xrow, first, end, acc);
 }
 
 // The expert passes of 8-row tiles (decode steps and the smallest chunks: an expert's one to eight rows). There are
@@ -344,18 +344,22 @@ __device__ __forceinline__ void small_walk(const MoeExpertArgs &a, SqMoeTileDesc
 // and a gate/up pass gives gate and up waves of their own: a workgroup's eight waves are the slices of the tensors of
 // 8 / (slices x tensors) column tiles, their sums meet in LDS in slice order. One launch runs the routed and the shared
 // tiles, each in its own format, so that the shared slices' long chains overlap the routed ones. 128 registers a wave
-// (chunks of two groups for the formats of more bits), so that two workgroups share a compute unit. Measured, 8 rows
-// over 256 experts of 2048 x 512 (Q4_K gate/up, Q5_K down, a Q8_0 shared slice): gate/up 40.6 us routed and 62.5 us
-// shared in two launches of whole-K waves -> 25 us; down 17.1 and 10.2 -> 17.5; at 170 registers 33 and 24.
-constexpr uint32_t kSmallWaves = 8;
-__global__ __launch_bounds__(64 * kSmallWaves) __attribute__((amdgpu_waves_per_eu(4)))
+// (chunks of two groups, the shortest that hold whole scale groups), so that four waves share a SIMD. A pass of one tensor
+// takes workgroups of four waves: a workgroup's registers and LDS are free again only when its last wave is done, and a
+// pass of many tiles runs in rounds of them. Measured, 8 rows over 256 experts of 2048 x 512 (Q4_K gate/up, Q5_K down, a
+// Q8_0 shared slice): gate/up 40.6 us routed and 62.5 us shared in two launches of whole-K waves -> 25 us; down 17.1 and
+// 10.2 -> 17.5; at 170 registers 33 and 24. The block of 16 / 32 rows over 256 af4g64 experts of 2048 x 512: whole-K waves
+// 64 / 87 us, eight waves and chunks of four groups 69 / 90, four waves in the down pass 66 / 87, and chunks of two 64 / 85;
+// one wave running its column tile's slices in turn took 90 / 129, gate and up (or two column tiles) in one wave 75 / 106.
+template <uint32_t WAVES>
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(4)))
 void expert_small_kernel(MoeExpertArgs a) {
   const uint32_t tile = blockIdx.y;
   if (tile >= a.tile_count->tiles) return;
   const SqMoeTileDescriptor d = a.tiles[tile];
   const int lane = threadIdx.x & 63, j = lane & 15, q = lane >> 4;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), tensors = a.gate_up ? 2 : 1;
-  const uint32_t per = kSmallWaves / (a.slices * tensors), ct0 = blockIdx.x * per;
+  const uint32_t per = WAVES / (a.slices * tensors), ct0 = blockIdx.x * per;
   const uint32_t column = wave / (a.slices * tensors), n = wave / a.slices % tensors, slice = wave % a.slices;
   const uint32_t column_tiles = a.output_size / 64, first_row = tile * a.tile_rows;
   float acc[1][4][1][4];
@@ -365,7 +369,7 @@ void expert_small_kernel(MoeExpertArgs a) {
     with_format(fmt, [&](auto f) { small_walk<decltype(f)::value>(a, d, first_row, n, ct0 + column, slice, acc); });
   }
   // red[wave][4 t + i][lane]: column block t, row 4 q + i.
-  __shared__ float red[kSmallWaves][16][64];
+  __shared__ float red[WAVES][16][64];
 #pragma unroll
   for (int t = 0; t < 4; ++t)
 #pragma unroll
@@ -376,7 +380,7 @@ void expert_small_kernel(MoeExpertArgs a) {
     for (uint32_t s = 0; s < a.slices; ++s) v += red[from + s][f][lane];
     return v;
   };
-  for (uint32_t o = wave; o < per * 16; o += kSmallWaves) {
+  for (uint32_t o = wave; o < per * 16; o += WAVES) {
     const uint32_t c = o / 16, f = o % 16, ct = ct0 + c, r = 4u * q + (f & 3), t = f >> 2;
     if (ct >= column_tiles || r >= d.rows) continue;
     // The gathering passes store at the column's place in the read order (chunk 4 g + j / 4 of its group, position
@@ -501,9 +505,9 @@ hipError_t launch_moe_expert_small(const MoeExpertArgs &args, hipStream_t stream
   // Slices of at least eight groups (the loads a wave keeps in flight) and at most four of them, in a power of two.
   const uint32_t spans = a.K / 32 / 4;
   a.slices = spans >= 8 ? 4 : spans >= 4 ? 2 : 1;
-  const uint32_t per = kSmallWaves / (a.slices * (a.gate_up ? 2 : 1));
-  hipLaunchKernelGGL(expert_small_kernel, dim3((a.output_size / 64 + per - 1) / per, a.max_tiles),
-                     dim3(64 * kSmallWaves), 0, stream, a);
+  const uint32_t waves = a.gate_up ? 8 : 4, per = waves / (a.slices * (a.gate_up ? 2 : 1));
+  hipLaunchKernelGGL(waves == 4 ? expert_small_kernel<4> : expert_small_kernel<8>,
+                     dim3((a.output_size / 64 + per - 1) / per, a.max_tiles), dim3(64 * waves), 0, stream, a);
   return hipGetLastError();
 }
 
