@@ -473,11 +473,13 @@ def test_row_tile_long_slices(fmt, rows, k):
 @pytest.mark.parametrize("fmt,rows,k", [(oracle.FMT_AF4G32, 17, 4352), (oracle.FMT_AF4G64, 32, 5120),
                                         (oracle.FMT_AF4G128, 20, 4608), (oracle.FMT_Q4K, 32, 5120),
                                         (oracle.FMT_Q4K, 31, 4352), (oracle.FMT_Q5K, 24, 4864),
-                                        (oracle.FMT_Q80, 24, 4352), (oracle.FMT_AF8G64, 32, 5120)])
+                                        (oracle.FMT_Q80, 24, 4352), (oracle.FMT_Q80, 24, 4800),
+                                        (oracle.FMT_AF8G64, 32, 5120)])
 def test_row_tile_slices_of_forty_groups(fmt, rows, k):
-    """17 to 32 rows past one round of workgroups (257 tiles): formats without plane1 bits run 129 to 160 groups as four
-    slices of 40, the last of 16 (K 4352) to 40 (K 5120) groups; Q5_K keeps slices of 32. Every
-    output against fp64 with the register tile's bound, and the last row's bits the same in 17 rows."""
+    """17 to 32 rows past one round of workgroups (257 tiles): 4-bit codes without plane1 bits run 129 to 160 groups as
+    four slices of 40, the last of 16 (K 4352) to 40 (K 5120) groups, 8-bit codes from 150 groups (K 4800) on; Q5_K and
+    shorter 8-bit ones keep slices of 32. Every output against fp64 with the register tile's bound, and the last row's
+    bits the same in 17 rows."""
     n = 64 * 257
     w = shape_weights(fmt, n, k, 23 + fmt)
     rng = np.random.default_rng(500 + rows + fmt + k)
@@ -487,6 +489,19 @@ def test_row_tile_slices_of_forty_groups(fmt, rows, k):
     check_decode(got, x, w, f"fmt {fmt} {n}x{k} rows {rows}")
     again = run_plan(staged(n, k, 17, 1), proj, x[-17:], n)
     assert np.array_equal(again[-1], got[-1])
+
+
+@pytest.mark.parametrize("fmt,k", [(oracle.FMT_Q80, 4352), (oracle.FMT_AF8G64, 4736)])
+def test_row_tile_eight_bit_slices(fmt, k):
+    """8-bit codes of 129 to 149 groups keep slices of 32 past one round of workgroups too (17 to 32 rows): the bits of
+    the same weights' first 200 tiles alone, which are within a round."""
+    n, few = 64 * 257, 64 * 200
+    w = shape_weights(fmt, n, k, 29 + fmt)
+    x = dense_inputs(np.random.default_rng(700 + k), 24, k)
+    got = run_plan(staged(n, k, 24, 1), sq.projection(w.segment()), x, n)
+    part = sq.segment(w.fmt, few, k, w.plane0, w.meta, 0, w.plane1)   # the planes are tile by tile
+    alone = run_plan(staged(few, k, 24, 1), sq.projection(part), x, few)
+    assert np.array_equal(got[:, :few], alone)
 
 
 NEW_FORMATS = [oracle.FMT_Q5K, oracle.FMT_Q6K, oracle.FMT_Q80, oracle.FMT_AF8G64]
