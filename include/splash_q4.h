@@ -91,7 +91,8 @@ typedef struct sq_linear_plan {
 
 /* LinearScratch / LinearScratchSize / LinearBuffers (runtime/ops/Linear.hpp:125-162,216-226). A decode plan's
  * partials hold its K splits' fp32 sums; a prefill plan's, where its tiles' K is halved (projections of 64 to 128
- * tiles of 256 rows by 256 columns, K a multiple of 512), the two halves' fp32 sums [2][rows][N], and where its
+ * tiles of 256 rows by 256 columns, K a multiple of 512; reserved there also where the narrow tile runs instead and
+ * leaves them untouched), the two halves' fp32 sums [2][rows][N], and where its
  * tiles number more than one round over the 256 compute units (K a multiple of 256), the fp32 sums of the last
  * round's stream pieces (128 MiB: two 256 x 256 tiles of sums for each of 256 workgroups) with a 4-byte counter
  * a stream tile. */
@@ -175,9 +176,9 @@ int sq_require_segment_planes(const sq_segment *segment, const char *what, uint3
  * projection of up to SQ_MAX_SEGMENTS segments runs them in one dispatch whatever their formats (gguf_decode_fused);
  * a prefill runs one dispatch per format. A prefill plan's input, output, residual, gate scratch, scratch table and
  * partials are 16-byte aligned and its row scales (scratch sums) 4-byte aligned. Whether a prefill halves its tiles'
- * K depends on the chunk's rows as well as the shape (a 4096-input, 14336-output projection halves from 257 to 512
- * rows), so a row's output bits may differ between chunks of different row counts; each lies within the row's fp64
- * interval. The same holds for the tiles past a prefill's whole rounds over the compute units, whose K runs in
+ * K, or runs its narrow tile (K in eight slices), depends on the chunk's rows as well as the shape (a 4096-input,
+ * 14336-output projection runs narrow up to 256 rows and halves from 257 to 512), so a row's output bits may differ
+ * between chunks of different row counts; each lies within the row's fp64 interval. The same holds for the tiles past a prefill's whole rounds over the compute units, whose K runs in
  * pieces on several workgroups (their sums add in K order whatever order the pieces finish in, so a chunk's bits
  * repeat from run to run). A decode row's bits depend only on the shape and the tile kind its rows run (1..4 rows,
  * 5..16, 17..32). */

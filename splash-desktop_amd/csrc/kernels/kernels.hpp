@@ -92,7 +92,7 @@ struct PrefillArgs {
   uint32_t stream_dp, stream_tiles, stream_range, stream_row_blocks;
 };
 hipError_t launch_prefill(uint32_t fmt, uint32_t epilogue, const PrefillArgs &args, hipStream_t stream);
-// The narrow tile's shape for a projection of `rows` x `plane_tiles` plane tiles (prefill_narrow.hip): 64 or 96 rows x 32
+// The narrow tile's shape for a dispatch of `rows` x `plane_tiles` plane tiles (prefill_narrow.hip): 64 or 96 rows x 32
 // or 64 columns a workgroup; rows 0 where the wide tile (prefill.hip) runs. `split`: the wide tile would halve its K.
 struct PrefillNarrow {
   uint32_t rows, columns;

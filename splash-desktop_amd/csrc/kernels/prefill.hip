@@ -956,27 +956,34 @@ PrefillSchedule prefill_schedule(uint32_t rows, uint32_t plane_tiles, uint32_t K
   if (7 * rounds128 < 10 * rounds256) return {128, 0, blocks128, columns, 0, 0};
   return {256, 0, blocks256, columns, 0, 0};
 }
-// The narrow tile's shape where its rounds of workgroups over the compute units cost less than the wide tile's, in
-// microseconds a 64-input step a round. Measured (Q4_K; the other formats' ratios are alike): 64 x 32 0.16-0.17, 64 x
-// 64 0.23-0.28, 96 x 32 0.21-0.23, 96 x 64 0.30-0.32 (128 x 32, 0.27-0.30, never costs less than 64 x 64); wide tiles
-// of 128 rows 1.03, of 256 1.87, halved 1.8 a step of a half and 15 for the close. The wide tile keeps what the narrow
-// one would not win by a twentieth. A function of the projection's whole width, so that every dispatch of it (one per
-// format) takes the same tile.
+// The narrow tile's shape where it costs less than the wide tile that would run (prefill_schedule). Costs in microseconds,
+// fitted to Q4_K over 431 shapes of 128..2048 rows, K 256..6144 and N 512..14336 whose two costs are near each other (rms
+// 4%): what a dispatch of either takes besides (kDispatch), a 64-input step of a round of workgroups, and what a round past
+// the first adds (the narrow tile's prologue, the sums of its slices and its stores, which the first round overlaps with
+// the dispatch). The wide tile keeps what the narrow one would not win by 8%. The other formats' costs keep
+// nearly these ratios (96 x 64 a step of the 128-row tile: Q4_K 0.26, the af4 ones 0.28, Q5_K 0.26, Q6_K 0.23, 8-bit codes
+// 0.24); over the same shapes in all eight the tile chosen was never more than 2% slower than the wide one, and on average
+// 0.6% slower than the fastest of the five. Without the rounds' own cost short K took the narrow tile where it loses: 2048
+// rows of K 1024 x N 2048 26 -> 30 us (af4g64; wide again 26), 1024 of K 256 x N 4096 13 -> 21. `plane_tiles` are the
+// dispatch's own: a projection of several formats runs a dispatch for each, and each pays its own rounds (512 rows of K
+// 5120, 7168 Q4_K and 1024 Q6_K columns: 170 us halved in two dispatches, 109 narrow).
 PrefillNarrow prefill_narrow(uint32_t rows, uint32_t plane_tiles, uint32_t K, bool split) {
-  const double steps = K / BK;
+  const double steps = K / BK, kDispatch = 9.0;
   const auto rounds = [&](uint32_t r, uint32_t c) {
-    return ((uint64_t)((rows + r - 1) / r) * ((plane_tiles * 64 + c - 1) / c) + kPrefillUnits - 1) / kPrefillUnits;
+    return (double)(((uint64_t)((rows + r - 1) / r) * ((plane_tiles * 64 + c - 1) / c) + kPrefillUnits - 1) / kPrefillUnits);
   };
-  const double wide = split ? 0.9 * steps + 15.0
-                            : steps * std::min(1.03 * (double)rounds(128, 256), 1.87 * (double)rounds(256, 256));
+  const PrefillSchedule sc = prefill_schedule(rows, plane_tiles, K, split);
+  const double wide = sc.split       ? 0.725 * steps + 16.0
+                      : sc.bm == 128 ? 0.995 * steps * rounds(128, 256)
+                                     : 1.55 * steps * rounds(256, 256) + 10.0 * (rounds(256, 256) - 1);
   struct {
     PrefillNarrow shape;
-    double cost;
-  } const shapes[] = {{{64, 32}, 0.165}, {{64, 64}, 0.26}, {{96, 32}, 0.22}, {{96, 64}, 0.31}};
+    double step, round;
+  } const shapes[] = {{{64, 32}, 0.131, 0.7}, {{64, 64}, 0.202, 3.2}, {{96, 32}, 0.185, 2.4}, {{96, 64}, 0.257, 4.2}};
   PrefillNarrow best{0, 0};
-  double least = 0.95 * wide;
+  double least = 0.92 * (wide + kDispatch) - kDispatch;
   for (const auto &s : shapes) {
-    const double cost = steps * s.cost * (double)rounds(s.shape.rows, s.shape.columns);
+    const double n = rounds(s.shape.rows, s.shape.columns), cost = n * steps * s.step + (n - 1) * s.round;
     if (cost < least) least = cost, best = s.shape;
   }
   return best;
@@ -1005,6 +1012,8 @@ PrefillStream prefill_stream(uint32_t row_blocks, uint32_t column_groups, uint32
   if (steps > 2 * range) return {0, 0, 0, 0};
   return {dp, stream, range, dp + row_blocks * ((work + range - 1) / range)};
 }
+// The halves' partials are reserved wherever the 256-row tiles would halve, also where every dispatch runs the narrow tile:
+// a plan's scratch, and so what a caller's scratch accepts and refuses, does not follow the measured costs.
 PrefillScratch prefill_scratch_bytes(uint32_t rows, uint32_t plane_tiles, uint32_t K) {
   if (prefill_split(rows, plane_tiles, K)) return {(uint64_t)2 * rows * ((plane_tiles + 3) / 4) * 256 * 4, 0};
   // A stream dispatch (any of the projection's, one a format, whose 256-row tiles are at most all of the
@@ -1030,8 +1039,9 @@ hipError_t launch_prefill_prepare(const uint16_t *input, uint32_t rows, uint32_t
 }
 
 hipError_t launch_prefill(uint32_t fmt, uint32_t epilogue, const PrefillArgs &a, hipStream_t stream) {
-  const uint32_t width = a.out_stride / 64;
-  const PrefillNarrow narrow = prefill_narrow(a.rows, width, a.K, prefill_split(a.rows, width, a.K));
+  uint32_t tiles = 0;
+  for (uint32_t s = 0; s < a.segments; ++s) tiles += a.seg[s].tiles;
+  const PrefillNarrow narrow = prefill_narrow(a.rows, tiles, a.K, prefill_split(a.rows, a.out_stride / 64, a.K));
   if (narrow.rows) return launch_prefill_narrow(fmt, epilogue, a, narrow, stream);
   switch (fmt) {
     case SQ_FMT_AF4G32: return launch_format<SQ_FMT_AF4G32>(epilogue, a, stream);

@@ -84,6 +84,57 @@ def test_prefill_tile_choice(fmt, rows, n, k):
     check_projection(run_prefill([w], x)[pick], x[pick], w, f"tile choice fmt {fmt}, {rows} rows of {k} x {n}")
 
 
+def prefill_tile(rows, n, k, own=None):
+    """The tile the library's rule picks for a dispatch of `own` columns of an n-column projection (all of them: one
+    format): "64x32" .. "96x64" (narrow), "wide128", "wide256" or "halved". Cases that are about one tile assert it."""
+    up = lambda a, b: -(-a // b)
+    own, steps = own or n, k // 64
+    rounds = lambda r, c, width: up(up(rows, r) * up(width, c), 256)
+    tiles256, tiles128 = up(rows, 256) * up(n, 256), up(rows, 128) * up(n, 256)
+    wide128, wide256 = rounds(128, 256, own), rounds(256, 256, own)
+    if 64 <= tiles256 <= 128 and steps % 8 == 0 and steps / 2 + 8 < min(0.7 * steps * up(tiles128, 256), steps):
+        tile, cost = "halved", 0.725 * steps + 16
+    elif 7 * wide128 < 10 * wide256:
+        tile, cost = "wide128", 0.995 * steps * wide128
+    else:
+        tile, cost = "wide256", 1.55 * steps * wide256 + 10 * (wide256 - 1)
+    cost = 0.92 * (cost + 9) - 9
+    for r, c, step, more in ((64, 32, 0.131, 0.7), (64, 64, 0.202, 3.2), (96, 32, 0.185, 2.4), (96, 64, 0.257, 4.2)):
+        count = rounds(r, c, own)
+        if count * steps * step + (count - 1) * more < cost:
+            tile, cost = f"{r}x{c}", count * steps * step + (count - 1) * more
+    return tile
+
+
+def test_prefill_short_k_runs_wide():
+    """K 1024, where the narrow tile's three rounds of workgroups cost more than a round of wide tiles: 2048 rows of 2048
+    columns give the bits of the same columns in a projection of 3072, far from the line."""
+    k, rows = 1024, 2048
+    assert prefill_tile(rows, 2048, k) == prefill_tile(rows, 3072, k) == "wide128"
+    rng = np.random.default_rng(81)
+    parts = [make_weights(rng, oracle.FMT_AF4G64, n, k) for n in (2048, 1024)]
+    x = dense_inputs(rng, rows, k)
+    alone = run_prefill(parts[:1], x)
+    assert np.array_equal(run_prefill(parts, x)[:, :2048], alone)
+    pick = sampled_rows(rows, 16, rng)
+    check_projection(alone[pick], x[pick], parts[0], "short K")
+
+
+def test_prefill_formats_take_tiles_of_their_own():
+    """A projection of two formats runs a dispatch for each, each on the tile its own columns take: the wide one, and the
+    narrow one that the same columns take alone (the same bits)."""
+    k, rows, ns = 512, 250, (14400, 192)
+    tiles = [prefill_tile(rows, sum(ns), k, n) for n in ns]
+    assert tiles == ["wide128", "64x32"] and prefill_tile(rows, 192, k) == "64x32"
+    rng = np.random.default_rng(82)
+    parts = [make_weights(rng, f, n, k) for f, n in zip((oracle.FMT_Q4K, oracle.FMT_Q6K), ns)]
+    x = dense_inputs(rng, rows, k)
+    out = run_prefill(parts, x)
+    assert np.array_equal(out[:, ns[0]:], run_prefill(parts[1:], x))
+    pick = sampled_rows(rows, 16, rng)
+    check_projection(out[pick], x[pick], parts, "tiles of their own")
+
+
 @pytest.mark.parametrize("k", [64, 448])
 def test_prefill_narrow_epilogues_and_segments(k):
     """The narrow tile under both epilogues and over a fused projection's segments, at K of one step and of seven."""
