@@ -108,17 +108,19 @@ void narrow_kernel(PrefillArgs a, uint32_t epilogue) {
     float *const cs = (float *)(xs + kRowBytes);   // (s, z) or half scales of [group][column]
     // The lane's column and (32 columns) its group of a step.
     const uint32_t col = NT == 4 ? lane : c0 + (lane & 31), half = NT == 4 ? 0u : lane >> 5;
-    // Buffer resources over the tile's planes and the rows (32-bit lane offsets, the step's offset scalar).
+    // Buffer resources over the tile's planes and the workgroup's own rows (32-bit lane offsets, the step's offset scalar;
+    // the extent of a whole chunk's rows would wrap from 4 GiB on, 2048 rows of K 2^20, and every load then read zeros).
+    const uint32_t live = min((uint32_t)BM, a.rows - row0);
     const auto planes = buffer_rsrc(seg.plane0 + (size_t)ptile * G * 64 * F::P0, G * 64 * F::P0);
     const auto metas = buffer_rsrc(seg.meta + (size_t)ptile * units * 64 * F::META, units * 64 * F::META);
     const auto highs = buffer_rsrc(F::P1 ? seg.plane1 + (size_t)ptile * G * 64 * F::P1 : nullptr, G * 64 * F::P1);
-    const auto rows = buffer_rsrc(a.half_input, a.rows * a.K * 2);
+    const auto rows = buffer_rsrc(a.half_input + (size_t)row0 * a.K, live * a.K * 2);
     const uint32_t pv = (half * 64 + col) * F::P0, hv = (c0 + j) * F::P1 + q * (F::P1 / 4);
     const uint32_t mv = (F::UNIT == 1 ? half * 64 + col : col) * F::META;
     uint32_t xv[XL];
 #pragma unroll
     for (int i = 0; i < XL; ++i)
-      xv[i] = min(row0 + 8 * i + (lane >> 3), a.rows - 1) * a.K * 2 + (lane & 7) * 16;
+      xv[i] = min(8u * i + (lane >> 3), live - 1) * a.K * 2 + (lane & 7) * 16;
     constexpr int CG = NT / 2;                            // code loads a step: groups a lane holds (1 or 2)
     constexpr int MU = NT == 4 && F::UNIT == 1 ? 2 : 1;   // meta units a lane reads a step
     u32x4 x[XL], codes[CG], codes_hi[F::P0 == 32 ? CG : 1];

@@ -135,6 +135,29 @@ def test_prefill_formats_take_tiles_of_their_own():
     check_projection(out[pick], x[pick], parts, "tiles of their own")
 
 
+def test_prefill_narrow_rows_of_four_gib():
+    """The narrow tile over a chunk whose fp16 rows are 4 GiB (2048 rows of K 2^20, one 64-column plane tile): rows of the
+    first, a middle and the last row block against fp64, within bf16's rounding and the sums' of fp32."""
+    t = torch()
+    rows, k, n = 2048, 1 << 20, 64
+    assert prefill_tile(rows, n, k) == "64x32" and rows * k * 2 == 1 << 32
+    w = DeviceAffine(np.random.default_rng(83), n, k)
+    gen = t.Generator(device="cuda").manual_seed(84)
+    x = t.empty((rows, k), dtype=t.bfloat16, device="cuda")
+    for at in range(0, rows, 64):
+        x[at:at + 64] = t.randn((64, k), device="cuda", generator=gen)
+    proj = sq.projection(w.segment())
+    plan = sq.plan_for(sq.prefill_workload(n, k, rows), proj)
+    scratch = sq.Scratch(plan)
+    out = t.empty((rows, n), dtype=t.bfloat16, device="cuda")
+    sq.linear_add(plan, proj, x, out, scratch=scratch.struct())
+    pick = [0, 63, 1000, 2047]
+    want = x[pick].double().cpu().numpy() @ w.values.astype(np.float64).T
+    got = out[pick].double().cpu().numpy()
+    # fp16 weights (2^-11), bf16 outputs (2^-9), fp32 sums (below 1e-5): as independent errors of each product, of the norm.
+    assert np.linalg.norm(got - want) <= 4e-3 * np.linalg.norm(want)
+
+
 @pytest.mark.parametrize("k", [64, 448])
 def test_prefill_narrow_epilogues_and_segments(k):
     """The narrow tile under both epilogues and over a fused projection's segments, at K of one step and of seven."""
