@@ -166,3 +166,25 @@ class Run:
 
     def output(self) -> np.ndarray:
         return to_host(self.out, self.out_dtype)
+
+
+def prefill_tile(rows, n, k, own=None):
+    """The tile the library's rule picks for a dispatch of `own` columns of an n-column projection (all of them: one
+    format): "64x32" .. "96x64" (narrow), "wide128", "wide256" or "halved". Cases that are about one tile assert it."""
+    up = lambda a, b: -(-a // b)
+    own, steps = own or n, k // 64
+    rounds = lambda r, c, width: up(up(rows, r) * up(width, c), 256)
+    tiles256, tiles128 = up(rows, 256) * up(n, 256), up(rows, 128) * up(n, 256)
+    wide128, wide256 = rounds(128, 256, own), rounds(256, 256, own)
+    if 64 <= tiles256 <= 128 and steps % 8 == 0 and steps / 2 + 8 < min(0.7 * steps * up(tiles128, 256), steps):
+        tile, cost = "halved", 0.725 * steps + 16
+    elif 7 * wide128 < 10 * wide256:
+        tile, cost = "wide128", 0.995 * steps * wide128
+    else:
+        tile, cost = "wide256", 1.55 * steps * wide256 + 10 * (wide256 - 1)
+    cost = 0.92 * (cost + 9) - 9
+    for r, c, step, more in ((64, 32, 0.131, 0.7), (64, 64, 0.202, 3.2), (96, 32, 0.185, 2.4), (96, 64, 0.257, 4.2)):
+        count = rounds(r, c, own)
+        if count * steps * step + (count - 1) * more < cost:
+            tile, cost = f"{r}x{c}", count * steps * step + (count - 1) * more
+    return tile

@@ -11,7 +11,7 @@ import pytest
 
 import splash_q4 as sq
 import sq_oracle as oracle
-from helpers import Run, dense_inputs, make_weights, to_device, torch
+from helpers import Run, dense_inputs, make_weights, prefill_tile, to_device, torch
 from splash_q4 import synthetic
 from test_moe_gpu import Block, make_plan
 
@@ -85,7 +85,8 @@ def test_graph_halved_prefill():
     proj = sq.projection(w.segment())
     plan = sq.plan_for(sq.prefill_workload(n, k, rows), proj)
     size, _ = sq.scratch_size(plan)
-    assert size.partials == 2 * rows * n * 4 and size.counters == 0, "the plan halves K"
+    assert size.partials == 2 * rows * n * 4 and size.counters == 0, "the plan reserves a halved K's sums"
+    assert prefill_tile(rows, n, k) == "halved"
     linear_case(plan, proj, n, rows, k, rng)
 
 

@@ -7,8 +7,8 @@ import pytest
 
 import splash_q4 as sq
 import sq_oracle as oracle
-from helpers import (DeviceAffine, Run, check_projection, dense_inputs, make_weights, sparse_inputs, staged_reference,
-                     to_device, torch)
+from helpers import (DeviceAffine, Run, check_projection, dense_inputs, make_weights, prefill_tile, sparse_inputs,
+                     staged_reference, to_device, torch)
 from splash_q4 import synthetic
 
 pytestmark = pytest.mark.gpu
@@ -23,7 +23,8 @@ def no_worse_than_staged(got, x, w, stats, what):
     assert stats["rel_l2"] <= ref_l2 * 1.10 + 1e-6, f"{what}: {stats['rel_l2']} against the staged {ref_l2}"
 
 
-def run_prefill(w_list, x, epilogue=sq.EPILOGUE_NONE, residual=None, gate_scratch=None, n=None):
+def run_prefill(w_list, x, epilogue=sq.EPILOGUE_NONE, residual=None, gate_scratch=None, n=None, halved=None):
+    """halved: whether the dispatch is to have halved its tiles' K, which writes the plan's partials."""
     segs, offset = [], 0
     for w in w_list:
         segs.append(w.segment(offset))
@@ -49,6 +50,10 @@ def run_prefill(w_list, x, epilogue=sq.EPILOGUE_NONE, residual=None, gate_scratc
     t.cuda.synchronize()
     out = run.output()
     assert np.all(out[rows:] == 0xFFFF), "rows past the chunk written"
+    if halved is not None:
+        assert sq.scratch_size(plan)[0].counters == 0, "partials of a halved K, not of stream pieces"
+        written = run.scratch.partials is not None and bool(run.scratch.partials.any())
+        assert written == halved, "the dispatch halves K" if halved else "the dispatch does not halve K"
     return out[:rows]
 
 
@@ -59,7 +64,7 @@ NEW_FORMATS = [oracle.FMT_Q5K, oracle.FMT_Q6K, oracle.FMT_Q80, oracle.FMT_AF8G64
 @pytest.mark.parametrize("rows", [33, 128, 300])
 def test_prefill_dense(fmt, rows):
     rng = np.random.default_rng(rows + fmt)
-    n, k = 320, 1024   # five 64-column tiles: the last workgroup's second half lies past the projection
+    n, k = 320, 1024   # ten workgroups of the narrow tile's 32 columns
     w = make_weights(rng, fmt, n, k)
     x = dense_inputs(rng, rows, k)
     stats = check_projection(run_prefill([w], x), x, w, f"prefill fmt {fmt} rows {rows}")
@@ -67,43 +72,22 @@ def test_prefill_dense(fmt, rows):
 
 
 @pytest.mark.parametrize("fmt", [oracle.FMT_AF4G64, oracle.FMT_Q4K, oracle.FMT_AF4G128, oracle.FMT_AF4G32] + NEW_FORMATS)
-@pytest.mark.parametrize("rows,n,k", [
-    (40, 1088, 768),      # 64 x 32: two or one steps a wave
-    (97, 2112, 1280),     # 64 x 32, a second row block of 33 rows, two or three steps a wave
-    (90, 5120, 512),      # 96 x 32, one step a wave
-    (128, 5120, 256),     # 64 x 64, half of the waves without steps
-    (200, 5120, 768),     # 96 x 64, the last row block of eight rows
-    (128, 27648, 512),    # 108 column groups: the wide tile of 128 rows
+@pytest.mark.parametrize("rows,n,k,tile", [
+    (40, 1088, 768, "64x32"),      # two or one steps a wave
+    (97, 2112, 1280, "64x32"),     # a second row block of 33 rows, two or three steps a wave
+    (90, 5120, 512, "96x32"),      # one step a wave
+    (128, 5120, 256, "64x64"),     # half of the waves without steps
+    (200, 5120, 768, "96x64"),     # the last row block of eight rows
+    (128, 27648, 512, "wide128"),  # 108 column groups
 ])
-def test_prefill_tile_choice(fmt, rows, n, k):
+def test_prefill_tile_choice(fmt, rows, n, k, tile):
     """The narrow tile's shapes and the wide tile beside them, at row and K remainders, against the fp64 interval."""
+    assert prefill_tile(rows, n, k) == tile
     rng = np.random.default_rng(rows + n + fmt)
     w = make_weights(rng, fmt, n, k)
     x = dense_inputs(rng, rows, k)
     pick = np.unique(np.r_[np.arange(0, rows, 11), rows - 1])
     check_projection(run_prefill([w], x)[pick], x[pick], w, f"tile choice fmt {fmt}, {rows} rows of {k} x {n}")
-
-
-def prefill_tile(rows, n, k, own=None):
-    """The tile the library's rule picks for a dispatch of `own` columns of an n-column projection (all of them: one
-    format): "64x32" .. "96x64" (narrow), "wide128", "wide256" or "halved". Cases that are about one tile assert it."""
-    up = lambda a, b: -(-a // b)
-    own, steps = own or n, k // 64
-    rounds = lambda r, c, width: up(up(rows, r) * up(width, c), 256)
-    tiles256, tiles128 = up(rows, 256) * up(n, 256), up(rows, 128) * up(n, 256)
-    wide128, wide256 = rounds(128, 256, own), rounds(256, 256, own)
-    if 64 <= tiles256 <= 128 and steps % 8 == 0 and steps / 2 + 8 < min(0.7 * steps * up(tiles128, 256), steps):
-        tile, cost = "halved", 0.725 * steps + 16
-    elif 7 * wide128 < 10 * wide256:
-        tile, cost = "wide128", 0.995 * steps * wide128
-    else:
-        tile, cost = "wide256", 1.55 * steps * wide256 + 10 * (wide256 - 1)
-    cost = 0.92 * (cost + 9) - 9
-    for r, c, step, more in ((64, 32, 0.131, 0.7), (64, 64, 0.202, 3.2), (96, 32, 0.185, 2.4), (96, 64, 0.257, 4.2)):
-        count = rounds(r, c, own)
-        if count * steps * step + (count - 1) * more < cost:
-            tile, cost = f"{r}x{c}", count * steps * step + (count - 1) * more
-    return tile
 
 
 def test_prefill_short_k_runs_wide():
@@ -177,6 +161,49 @@ def test_prefill_narrow_epilogues_and_segments(k):
     want = synthetic.bf16_to_f32(plain).astype(np.float64) * gf / (1 + np.exp(-gf))
     ulp = np.ldexp(1.0, np.floor(np.log2(np.maximum(np.abs(want), 1e-30))).astype(int) - 7)
     assert np.all(np.abs(got - want) <= ulp + 1e-30)
+
+
+@pytest.mark.parametrize("fmt", [oracle.FMT_Q4K, oracle.FMT_Q6K, oracle.FMT_Q80])
+@pytest.mark.parametrize("rows,tile", [(250, "wide128"), (600, "wide256")])
+def test_prefill_wide_ragged_columns(fmt, rows, tile):
+    """The wide tiles (eight waves, Q4_K, and four) at one 64-column plane tile past whole groups of 256 columns and a
+    ragged last row block: plain, with the residual and the up-with-gate epilogues, and over segments that meet inside a
+    group."""
+    n, k = 14400, 512
+    assert prefill_tile(rows, n, k) == tile
+    rng = np.random.default_rng(85 + fmt + rows)
+    parts = [make_weights(rng, fmt, m, k) for m in (8256, 64, 6080)]
+    x = dense_inputs(rng, rows, k)
+    pick = sampled_rows(rows, 12, rng)
+    check_projection(run_prefill(parts, x)[pick], x[pick], parts, f"{tile} segments fmt {fmt}")
+    w = make_weights(rng, fmt, n, k)
+    plain = run_prefill([w], x)
+    check_projection(plain[pick], x[pick], w, f"{tile} fmt {fmt}")
+    residual = synthetic.bf16_bits(rng.uniform(-64, 64, (rows, n)).astype(np.float32))
+    out = run_prefill([w], x, sq.EPILOGUE_RESIDUAL, residual=residual)
+    check_projection(out[pick], x[pick], w, f"{tile} residual fmt {fmt}", residual=residual[pick])
+    gate = synthetic.bf16_bits(rng.uniform(-4, 4, (rows, n)).astype(np.float32))
+    got = run_prefill([w], x, sq.EPILOGUE_UP_WITH_GATE, gate_scratch=gate)[pick]
+    gf = synthetic.bf16_to_f32(gate[pick]).astype(np.float64)
+    want = synthetic.bf16_to_f32(plain[pick]).astype(np.float64) * gf / (1 + np.exp(-gf))
+    ulp = np.ldexp(1.0, np.floor(np.log2(np.maximum(np.abs(want), 1e-30))).astype(int) - 7)
+    assert np.all(np.abs(synthetic.bf16_to_f32(got).astype(np.float64) - want) <= ulp + 1e-30)
+
+
+@pytest.mark.parametrize("rows", [128, 300])
+def test_prefill_wide_sparse_and_mixed_rows(rows):
+    """The wide tiles' row scales: +-1e5 alone, and beside values of 1e-3."""
+    n, k = 20480, 256
+    assert prefill_tile(rows, n, k).startswith("wide")
+    rng = np.random.default_rng(86 + rows)
+    w = make_weights(rng, oracle.FMT_AF4G64, n, k)
+    pick = sampled_rows(rows, 12, rng)
+    x = sparse_inputs(rows, k)
+    check_projection(run_prefill([w], x)[pick], x[pick], w, "wide sparse")
+    xm = synthetic.bf16_to_f32(dense_inputs(rng, rows, k)) * np.float32(1e-3)
+    xm[:, ::100] = 1e5
+    xb = synthetic.bf16_bits(xm)
+    check_projection(run_prefill([w], xb)[pick], xb[pick], w, "wide mixed")
 
 
 def test_prefill_sparse_inputs_past_half_range():
@@ -362,19 +389,20 @@ def test_config2_ragged_with_small_rows():
 
 def test_prefill_halving_depends_on_the_chunk_rows():
     """Whether the prefill halves its tiles' K depends on the chunk's rows as well as the shape (4096 x 14336 halves
-    from 257 to 512 rows, not at 256), so a row's bits can differ between chunks of 256 and 257 rows; both lie
-    inside the row's fp64 interval, and their difference within two fp32 accumulation bounds of it."""
+    from 257 to 512 rows, runs narrow up to 256 and whole tiles from 513), so a row's bits can differ between chunks of
+    512 and 513 rows; both lie inside the row's fp64 interval, and their difference within two fp32 accumulation bounds
+    of it."""
     n, k = 14336, 4096
     w = shape_weights(oracle.FMT_AF4G64, n, k, n + k)
-    proj = sq.projection(w.segment())
-    halved = lambda r: sq.scratch_size(sq.plan_for(sq.prefill_workload(n, k, r), proj))[0].partials > 0
-    assert not halved(256) and halved(257)
+    assert [prefill_tile(r, n, k) for r in (256, 257, 512, 513)] == ["96x64", "halved", "halved", "wide256"]
     rng = np.random.default_rng(257)
-    x = dense_inputs(rng, 257, k)
-    whole, cut = run_prefill([w], x[:256]), run_prefill([w], x)[:256]
-    pick = np.arange(0, 256, 17)
-    check_projection(whole[pick], x[pick], w, "256 rows, whole K")
-    check_projection(cut[pick], x[pick], w, "257 rows, halved K")
+    x = dense_inputs(rng, 513, k)
+    run_prefill([w], x[:256], halved=False)
+    run_prefill([w], x[:257], halved=True)
+    whole, cut = run_prefill([w], x, halved=False)[:512], run_prefill([w], x[:512], halved=True)
+    pick = np.arange(0, 512, 33)
+    check_projection(whole[pick], x[pick], w, "513 rows, whole K")
+    check_projection(cut[pick], x[pick], w, "512 rows, halved K")
     value, magnitude, inputs, largest = oracle.project_f64(x[pick], w.values)
     bound = 2 * oracle.projection_bound(magnitude, inputs, largest, True) + \
         oracle.ulp_bf16(np.maximum(np.abs(value), 1e-30))
@@ -394,7 +422,7 @@ def test_prefill_halved_k(fmt):
     assert size.partials == 2 * rows * n * 4, "the plan halves K"
     rng = np.random.default_rng(71 + fmt)
     x = dense_inputs(rng, rows, k)
-    out = run_prefill([w], x)
+    out = run_prefill([w], x, halved=True)
     check_sampled(out, x, w, f"halved K fmt {fmt}", rng)
 
 
@@ -412,7 +440,7 @@ def test_prefill_halved_k_across_segments():
     size, _ = sq.scratch_size(sq.plan_for(sq.prefill_workload(n, k, rows), sq.projection(segs)))
     assert size.partials == 2 * rows * n * 4, "the plan halves K"
     x = dense_inputs(rng, rows, k)
-    out = run_prefill(parts, x)
+    out = run_prefill(parts, x, halved=True)
     pick = sampled_rows(rows, 24, rng)
     check_projection(out[pick], x[pick], parts, "halved K across segments")
 
@@ -426,8 +454,9 @@ def test_prefill_halved_k_mixed_formats():
     segs = [parts[0].segment(0), parts[1].segment(4096)]
     size, _ = sq.scratch_size(sq.plan_for(sq.prefill_workload(8192, k, rows), sq.projection(segs)))
     assert size.partials == 2 * rows * 8192 * 4, "the plan halves K"
+    assert prefill_tile(rows, 8192, k, 4096) == "halved"
     x = dense_inputs(rng, rows, k)
-    out = run_prefill(parts, x)
+    out = run_prefill(parts, x, halved=True)
     pick = sampled_rows(rows, 24, rng)
     check_projection(out[pick], x[pick], parts, "halved K, two formats")
 
@@ -439,9 +468,9 @@ def test_prefill_halved_k_epilogues():
     w = make_weights(rng, oracle.FMT_AF4G64, n, k)
     x = dense_inputs(rng, rows, k)
     pick = sampled_rows(rows, 24, rng)
-    plain = run_prefill([w], x)
+    plain = run_prefill([w], x, halved=True)
     residual = synthetic.bf16_bits(rng.uniform(-64, 64, (rows, n)).astype(np.float32))
-    out = run_prefill([w], x, sq.EPILOGUE_RESIDUAL, residual=residual)
+    out = run_prefill([w], x, sq.EPILOGUE_RESIDUAL, residual=residual, halved=True)
     check_projection(out[pick], x[pick], w, "halved residual", residual=residual[pick])
     gate = synthetic.bf16_bits(rng.uniform(-4, 4, (rows, n)).astype(np.float32))
     up_gated = run_prefill([w], x, sq.EPILOGUE_UP_WITH_GATE, gate_scratch=gate)

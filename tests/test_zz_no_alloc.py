@@ -112,9 +112,10 @@ def test_static_epilogue_operands_then_smaller():
 
 
 def test_static_halved_prefill_then_smaller():
-    """A prefill whose tiles' K is halved (16384 x 3072 at 40 rows, then 33: 64 tiles of 256 columns, each cut
-    between two workgroups whose fp32 halves a close dispatch adds) takes its partials from the static array: bitwise
-    sq_linear_add's."""
+    """A prefill whose plan reserves the partials of a halved K (16384 x 3072 at 40 rows, then 33: 64 tiles of 256
+    columns) takes them from the static array, though its dispatch runs the narrow tile and leaves them untouched:
+    bitwise sq_linear_add's. (No plan that fits the array halves: from 64 tiles of 256 columns on, its partials leave
+    room for the row counts of the narrow tile only.)"""
     rng = np.random.default_rng(76)
     n, k = 16384, 3072
     w = DeviceAffine(rng, n, k)
@@ -122,7 +123,7 @@ def test_static_halved_prefill_then_smaller():
     for rows in (40, 33):
         plan = sq.plan_for(sq.prefill_workload(n, k, rows), proj)
         size, _ = sq.scratch_size(plan)
-        assert plan.config.tile == sq.TILE_PREFILL and size.partials == 2 * rows * n * 4, "the plan halves K"
+        assert plan.config.tile == sq.TILE_PREFILL and size.partials == 2 * rows * n * 4, "the plan reserves halves"
         x = dense_inputs(rng, rows, k)
         want, got = run_both(plan, proj, x, n)
         assert np.array_equal(got, want), rows
