@@ -221,7 +221,7 @@ def check_block(block, x, scores, top_k, residual, phase="prefill", weight_rtol=
                                  oracle.FMT_AF8G64])
 @pytest.mark.parametrize("rows", [40, 6])
 def test_moe_routed_formats(fmt, rows):
-    """Every format through both expert-pass register budgets (tiles of 32 and of 16 rows)."""
+    """Every format through both expert passes (32-row tiles, and the 8-row ones of a decode step)."""
     rng = np.random.default_rng(900 + fmt + rows)
     block = Block(rng, 16, 512, 256, fmt=fmt)
     x = synthetic.activations(rng, rows, 512)
@@ -250,7 +250,7 @@ def test_moe_small_tile_slices(fmt, hidden, inner):
                                  oracle.FMT_Q4K, oracle.FMT_Q5K, oracle.FMT_Q6K, oracle.FMT_Q80])
 @pytest.mark.parametrize("rows,hidden,inner", [
     (150, 1024, 256),    # gate/up from the sorted work list, down by tile; experts of one to four tiles
-    (75, 256, 1280),   # gate/up by tile, down from the list; column groups short of a workgroup's
+    (75, 256, 1280),   # gate/up by tile, down from the list
 ])
 def test_moe_tile_pairs(fmt, rows, hidden, inner):
     """32-row tiles two of an expert at a time: experts of odd and even tile counts, short last tiles, both ways a
@@ -262,6 +262,25 @@ def test_moe_tile_pairs(fmt, rows, hidden, inner):
     scores = synthetic.router_logits(rng, rows, 6)
     scores[:, 0] += 3   # the first expert takes nearly every row
     check_block(block, x, scores, 2, None)
+
+
+@pytest.mark.parametrize("rows,hidden,inner,formats", [
+    (75, 256, 192, {}),                                  # six 32-column blocks of gate and up over waves of four
+    (40, 512, 320, {"up": oracle.FMT_AF4G32}),           # a gate pass and an up pass: ten blocks over waves of eight
+    (90, 1024, 320, {"gate": oracle.FMT_Q4K, "up": oracle.FMT_Q4K}),
+    (75, 256, 192, {"gate": oracle.FMT_Q6K, "up": oracle.FMT_Q5K, "down": oracle.FMT_Q80}),
+])
+def test_moe_wide_spare_waves(rows, hidden, inner, formats):
+    """32-row tiles whose column blocks leave waves of the last group spare (they walk the last block, keep the barriers
+    and store nothing): one-pass pairs and a gate and an up of different formats, the shared slice's likewise, tiles
+    alone and two to a workgroup."""
+    rng = np.random.default_rng(1900 + hidden + inner)
+    block = Block(rng, 6, hidden, inner, shared=1, gated=True, shared_fmt=oracle.FMT_AF8G64, formats=formats)
+    x = synthetic.activations(rng, rows, hidden)
+    scores = synthetic.router_logits(rng, rows, 6)
+    scores[:, 0] += 3
+    _, tiles, _ = check_block(block, x, scores, 2, None)
+    assert tiles[:, 1].max() == 32
 
 
 @pytest.mark.parametrize("fmt,inner", [(oracle.FMT_AF4G32, 64), (oracle.FMT_AF4G64, 320), (oracle.FMT_AF4G128, 384),
@@ -314,9 +333,8 @@ def test_moe_35b_formats():
 
 
 def test_moe_rows_independent_of_the_block():
-    """A row's output is bitwise the same in any block: the 35B mix (its gated Q8_0 shared slice in launches of its
-    own, whose few tiles run as 16-row halves) over 70 rows and over their first 24 (other expert tiles, other
-    halves)."""
+    """A row's output is bitwise the same in any block of 32-row tiles: the 35B mix (its gated Q8_0 shared slice in
+    launches of its own, each tile alone) over 70 rows and over their first 24 (other expert tiles)."""
     rng = np.random.default_rng(991)
     block = Block(rng, 32, 512, 256, fmt=oracle.FMT_Q4K, shared=1, gated=True, shared_fmt=oracle.FMT_Q80,
                   formats={"down": oracle.FMT_Q5K})
@@ -492,8 +510,8 @@ def test_moe_verify_rows(shared):
 @pytest.mark.parametrize("fmt", [oracle.FMT_AF4G64, oracle.FMT_AF4G32, oracle.FMT_AF4G128, oracle.FMT_Q4K,
                                  oracle.FMT_Q5K, oracle.FMT_Q6K, oracle.FMT_Q80, oracle.FMT_AF8G64])
 def test_moe_tall_tiles_every_format(fmt):
-    """Router scores skewed towards four experts give them tiles of more than 16 rows (the two-row-block body of the
-    expert passes), in every format, in the one-pass gate/up pair (two tensors a wave) and the down pass (one)."""
+    """Router scores skewed towards four experts give them tiles of more than 16 rows, two of some of them to a
+    workgroup, in every format, in the one-pass gate/up pair and the down pass."""
     rng = np.random.default_rng(1300 + fmt)
     block = Block(rng, 16, 512, 256, fmt=fmt)
     rows = 64
@@ -506,8 +524,8 @@ def test_moe_tall_tiles_every_format(fmt):
 
 def test_moe_config4_block():
     """BASELINE config 4 at full size: 128 experts, top 8 of softmax(N(0,1) logits), hidden 2048, intermediate 768,
-    512 tokens, MLX affine 4-bit group 64, on the prefill plan (32-row tiles, about 250 of them, dispatched longest
-    first). Every row of the output against fp64 within BASELINE's tolerances, and no worse than the reference's
+    512 tokens, MLX affine 4-bit group 64, on the prefill plan (32-row tiles, about 250 of them, two of an expert to a
+    workgroup, pairs first). Every row of the output against fp64 within BASELINE's tolerances, and no worse than the reference's
     staged expert numerics emulated on the CPU."""
     rng = np.random.default_rng(4096)
     block = Block(rng, 128, 2048, 768, device_repack=True)
