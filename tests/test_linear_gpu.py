@@ -491,6 +491,39 @@ def test_row_tile_slices_of_forty_groups(fmt, rows, k):
     assert np.array_equal(again[-1], got[-1])
 
 
+@pytest.mark.parametrize("fmt", [oracle.FMT_Q4K, oracle.FMT_Q80])
+def test_row_tile_slices_of_forty_groups_outputs(fmt):
+    """The slices of 40 groups with the residual epilogue against fp64, and with fp32 outputs, which round to the plain
+    ones."""
+    n, k, rows = 64 * 257, 4864, 20
+    w = shape_weights(fmt, n, k, 31 + fmt)
+    rng = np.random.default_rng(600 + fmt)
+    x = dense_inputs(rng, rows, k)
+    residual = synthetic.bf16_bits(rng.uniform(-64, 64, (rows, n)).astype(np.float32))
+    got = run_plan(staged(n, k, rows, 1, sq.EPILOGUE_RESIDUAL), sq.projection(w.segment()), x, n, residual=residual)
+    check_decode(got, x, w, f"fmt {fmt} residual", residual=residual)
+    plain = run_plan(staged(n, k, rows, 1), sq.projection(w.segment()), x, n)
+    f32 = run_plan(staged(n, k, rows, 1, destination=sq.OUTPUT_F32), sq.projection(w.segment(), destination=sq.OUTPUT_F32),
+                   x, n, np.float32)
+    assert np.array_equal(synthetic.bf16_bits(f32), plain)
+
+
+@pytest.mark.parametrize("formats", [(oracle.FMT_Q4K, oracle.FMT_Q6K), (oracle.FMT_Q6K, oracle.FMT_Q4K)])
+def test_row_tile_mixed_formats_past_a_round(formats):
+    """Mixed segments past one round of workgroups keep slices of 32 groups where a projection of one format takes 40 (K
+    5120, 20 rows): against fp64, and the bits of each segment alone within a round, whose slices are 32 as well."""
+    k, rows, ns = 5120, 20, (64 * 200, 64 * 57)
+    rng = np.random.default_rng(610 + formats[0])
+    parts = [make_weights(rng, f, n, k) for f, n in zip(formats, ns)]
+    x = dense_inputs(rng, rows, k)
+    segs = [parts[0].segment(0), parts[1].segment(ns[0])]
+    fused = run_plan(staged(sum(ns), k, rows, 1), sq.projection(segs), x, sum(ns))
+    check_decode(fused, x, parts, f"mixed {formats}")
+    for p, at in zip(parts, (0, ns[0])):
+        alone = run_plan(staged(p.n, k, rows, 1), sq.projection(p.segment()), x, p.n)
+        assert np.array_equal(fused[:, at:at + p.n], alone), f"segment at {at} ({p.fmt})"
+
+
 @pytest.mark.parametrize("fmt,k", [(oracle.FMT_Q80, 4352), (oracle.FMT_AF8G64, 4736)])
 def test_row_tile_eight_bit_slices(fmt, k):
     """8-bit codes of 129 to 149 groups keep slices of 32 past one round of workgroups too (17 to 32 rows): the bits of
