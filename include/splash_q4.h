@@ -178,10 +178,10 @@ int sq_require_segment_planes(const sq_segment *segment, const char *what, uint3
  * partials are 16-byte aligned and its row scales (scratch sums) 4-byte aligned. Whether a prefill halves its tiles'
  * K, or runs its narrow tile (K in eight slices), depends on the chunk's rows as well as the shape (a 4096-input,
  * 14336-output projection runs narrow up to 256 rows and halves from 257 to 512), so a row's output bits may differ
- * between chunks of different row counts; each lies within the row's fp64 interval. The same holds for the tiles past a prefill's whole rounds over the compute units, whose K runs in
- * pieces on several workgroups (their sums add in K order whatever order the pieces finish in, so a chunk's bits
- * repeat from run to run). A decode row's bits depend only on the shape and the tile kind its rows run (1..4 rows,
- * 5..16, 17..32). */
+ * between chunks of different row counts; each lies within the row's fp64 interval. The same holds for the tiles past
+ * a prefill's whole rounds over the compute units, whose K runs in pieces on several workgroups (their sums add in K
+ * order whatever order the pieces finish in, so a chunk's bits repeat from run to run). A decode row's bits depend only
+ * on the shape, the segments' formats and the tile kind its rows run (1..4 rows, 5..16, 17..32). */
 int sq_linear_add(void *graph, const sq_linear_buffers *buffers, const sq_projection *projection,
                   const sq_linear_plan *plan, const sq_projection *gate);
 /* Linear::add with its result: *prepared (may be NULL) receives what the scratch table describes after the

@@ -267,13 +267,13 @@ DecodeLayout decode_layout(uint32_t fmt, uint32_t blocks, uint32_t K, uint32_t s
   // Past one round of workgroups, 32 rows of one tensor whose slices of 32 groups would be five waves take four of 40:
   // the fifth wave doubles up on the first SIMD, and a second workgroup's would need four waves' registers there, so a
   // compute unit held one workgroup where four waves leave room for two. 8-bit codes take them from kWideBytes32 groups
-  // on: below, five shorter waves, which issue more, are done sooner. Measured, five of 32 -> four of 40 (N 17408, K 4352
-  // / 4608 / 4800 / 4864 / 5120): Q4_K at 17 rows 31.4 / 31.2 / - / 32.6 / 37.2 -> 26.4 / 25.6 / - / 25.8 / 26.0 us, at
-  // 32 rows 32.9 / 32.7 / - / 33.6 / 39.5 -> 33.2 / 31.7 / - / 31.9 / 34.4; af4g64 at 32 rows 31.5 / 31.0 / 30.9 / 30.9 /
-  // 36.0 -> 31.5 / 30.7 / 31.5 / 30.9 / 33.8; Q8_0 at 17 rows 39.7 / 38.8 / 41.1 / 42.8 / 49.4 -> 41.3 / 40.4 / 40.3 /
-  // 40.7 / 42.0, at 32 rows 46.4 / 45.8 / 47.5 / 48.8 / 56.1 -> 48.3 / 47.2 / 47.5 / 47.3 / 49.9, and the same in two and
-  // four splits of as many groups. With plane1 bits the longer slice spills (Q6_K, K 5120, 67.6 -> 138.6), so those
-  // formats keep 32, and mixed segments with them (launch_decode).
+  // on: below, five shorter waves, which issue more, are done sooner. Measured, five of 32 -> four of 40 (N 17408, K
+  // 4352 / 4608 / 4800 / 4864 / 5120): Q4_K at 17 rows 31.4 / 31.2 / - / 32.6 / 37.2 -> 26.4 / 25.6 / - / 25.8 / 26.0
+  // us, at 32 rows 32.9 / 32.7 / - / 33.6 / 39.5 -> 33.2 / 31.7 / - / 31.9 / 34.4; af4g64 at 32 rows 31.5 / 31.0 / 30.9
+  // / 30.9 / 36.0 -> 31.5 / 30.7 / 31.5 / 30.9 / 33.8; Q8_0 at 17 rows 39.7 / 38.8 / 41.1 / 42.8 / 49.4 -> 41.3 / 40.4
+  // / 40.3 / 40.7 / 42.0, at 32 rows 46.4 / 45.8 / 47.5 / 48.8 / 56.1 -> 48.3 / 47.2 / 47.5 / 47.3 / 49.9, and the same
+  // in two and four splits of as many groups. With plane1 bits the longer slice spills (Q6_K, K 5120, 67.6 -> 138.6),
+  // so those formats keep 32, and mixed segments with them (launch_decode).
   const bool bytes32 = sq_format(fmt).plane0_bytes == 32;
   if (rows > 16 && !pair && !sq_format(fmt).plane1_bytes && tiles * splits > kDecodeUnits &&
       gs > (bytes32 ? kWideBytes32 - 1 : 4 * kColumnMaxGroups) && gs <= kWideWaves * kWideGroups)
@@ -304,9 +304,9 @@ hipError_t launch_decode(uint32_t fmt, uint32_t epilogue, bool f32_output, const
   const bool pair = args.gate.plane0 != nullptr;
   DecodeLayout layout = decode_layout(layout_format(fmt, args), tiles * 4, args.K, args.splits, pair, args.rows);
   if (!layout.nb) return hipErrorInvalidValue;
-  // Segments of mixed formats keep five slices of 32 over the same 129 to 160 groups: their kernel walks every format in
-  // one instance, and the formats with plane1 bits spill in slices of 40. So there a segment's sums run in another order
-  // than in a projection of its own format.
+  // Segments of mixed formats keep five slices of 32 over the same 129 to 160 groups: their kernel walks every format
+  // in one instance, and the formats with plane1 bits spill in slices of 40. So there a segment's sums run in another
+  // order than in a projection of its own format.
   if (fmt == kSegmentFormats && layout.ks == kWideGroups) layout = {5, kColumnMaxGroups};
   switch (fmt) {
     case SQ_FMT_AF4G32: return launch_format<SQ_FMT_AF4G32>(epilogue, f32_output, pair, args, tiles, layout, stream);

@@ -329,28 +329,29 @@ __device__ __forceinline__ void small_walk(const MoeExpertArgs &a, SqMoeTileDesc
   if (first >= end) return;
   const bool shared = d.expert >= a.experts;
   const size_t pt = (size_t)(shared ? d.expert - a.experts : a.slots[d.expert]) * (a.output_size / 64) + ct;
-  const uint8_t *const plane[1] = {(shared ? a.shared_plane0[n] : a.plane0[n]) + (pt * G * 64 + lane) * F::P0};
-  const uint8_t *const high[1] = {
-      F::P1 ? (shared ? a.shared_plane1[n] : a.plane1[n]) + (pt * G * 64 + lane) * F::P1 : nullptr};
-  const uint8_t *const meta[1] = {(shared ? a.shared_meta[n] : a.meta[n]) + (pt * (G / F::UNIT) * 64 + lane) * F::META};
+  const uint8_t *const plane = (shared ? a.shared_plane0[n] : a.plane0[n]) + (pt * G * 64 + lane) * F::P0;
+  const uint8_t *const high =
+      F::P1 ? (shared ? a.shared_plane1[n] : a.plane1[n]) + (pt * G * 64 + lane) * F::P1 : nullptr;
+  const uint8_t *const meta = (shared ? a.shared_meta[n] : a.meta[n]) + (pt * (G / F::UNIT) * 64 + lane) * F::META;
   const uint32_t r = (uint32_t)j < d.rows ? j : 0u;
   const uint32_t source = a.gather ? a.routes[first_row + r] / a.routes_per_row : first_row + r;
-  const uint16_t *const xrow[1] = {a.input + (size_t)source * a.K + 8 * q};
-  row_stream<FMT, 1, 1, 2, F::SG <= 2 ? 2 : 4>(plane, high, meta, xrow, first, end, acc);
+  const uint16_t *const xrow = a.input + (size_t)source * a.K + 8 * q;
+  row_stream<FMT, F::SG <= 2 ? 2 : 4>(plane, high, meta, xrow, first, end, acc);
 }
 
-// The expert passes of 8-row tiles (decode steps and the smallest chunks: an expert's one to eight rows). There are
-// few tiles and each wave's walk over K is a chain of loads it waits on, so K is cut into `slices` slices, a wave each,
-// and a gate/up pass gives gate and up waves of their own: a workgroup's eight waves are the slices of the tensors of
-// 8 / (slices x tensors) column tiles, their sums meet in LDS in slice order. One launch runs the routed and the shared
+// The expert passes of 8-row tiles (decode steps and the smallest chunks: an expert's one to eight rows). There are few
+// tiles and each wave's walk over K is a chain of loads it waits on, so K is cut into `slices` slices, a wave each, and
+// a gate/up pass gives gate and up waves of their own: a workgroup's eight waves are the slices of the tensors of 8 /
+// (slices x tensors) column tiles, their sums meet in LDS in slice order. One launch runs the routed and the shared
 // tiles, each in its own format, so that the shared slices' long chains overlap the routed ones. 128 registers a wave
-// (chunks of two groups, the shortest that hold whole scale groups), so that four waves share a SIMD. A pass of one tensor
-// takes workgroups of four waves: a workgroup's registers and LDS are free again only when its last wave is done, and a
-// pass of many tiles runs in rounds of them. Measured, 8 rows over 256 experts of 2048 x 512 (Q4_K gate/up, Q5_K down, a
-// Q8_0 shared slice): gate/up 40.6 us routed and 62.5 us shared in two launches of whole-K waves -> 25 us; down 17.1 and
-// 10.2 -> 17.5; at 170 registers 33 and 24. The block of 16 / 32 rows over 256 af4g64 experts of 2048 x 512: whole-K waves
-// 64 / 87 us, eight waves and chunks of four groups 69 / 90, four waves in the down pass 66 / 87, and chunks of two 64 / 85;
-// one wave running its column tile's slices in turn took 90 / 129, gate and up (or two column tiles) in one wave 75 / 106.
+// (chunks of two groups, the shortest that hold whole scale groups), so that four waves share a SIMD. A pass of one
+// tensor takes workgroups of four waves: a workgroup's registers and LDS are free again only when its last wave is
+// done, and a pass of many tiles runs in rounds of them. Measured, 8 rows over 256 experts of 2048 x 512 (Q4_K gate/up,
+// Q5_K down, a Q8_0 shared slice): gate/up 40.6 us routed and 62.5 us shared in two launches of whole-K waves -> 25 us;
+// down 17.1 and 10.2 -> 17.5; at 170 registers 33 and 24. The block of 16 / 32 rows over 256 af4g64 experts of 2048 x
+// 512: whole-K waves 64 / 87 us, eight waves and chunks of four groups 69 / 90, four waves in the down pass 66 / 87,
+// and chunks of two 64 / 85; one wave running its column tile's slices in turn took 90 / 129, gate and up (or two
+// column tiles) in one wave 75 / 106.
 template <uint32_t WAVES>
 __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(4)))
 void expert_small_kernel(MoeExpertArgs a) {

@@ -6,14 +6,14 @@
 // streams 32 columns of one tensor over all of K (a gate/up pass: waves 0..3 gate, 4..7 up of the same columns, which
 // meet in LDS at the end), 128 registers, so four waves share a SIMD and cover each other's dependency stalls (a wave
 // of both tensors' 32 columns, two a SIMD, took 206 us where this takes 160: Q4_K gate/up of 1999 rows of 8 routes over
-// 256 experts of 2048 x 512; the row tile's 16x16x32 walk of 32 rows, 213; VALU issue 55% of the dispatch). Per step of 64 inputs
+// 256 experts of 2048 x 512; the row tile's 16x16x32 walk of 32 rows, 213). Per step of 64 inputs
 //  - the workgroup's rows come 128 bytes a row (eight lanes a row, whole cache lines) through registers into LDS, one
-//    step ahead (32 rows and fewer: two), in two stages with one barrier each, with each group's input sums (four lanes a
-//    group) beside them; every wave reads its MFMA fragments from there;
+//    step ahead (32 rows and fewer: two), in two stages with one barrier each, with each group's input sums (four lanes
+//    a group) beside them; every wave reads its MFMA fragments from there;
 //  - a lane holds one column's codes of one of the step's groups (lane l: column l % 32, group l / 32), so two
 //    v_permlane32_swap turn a block's words into both groups' B operands, the lane derives one (column, group)'s
-//    coefficients, one more swap gives every lane its column's scales of both groups, and the offsets already lie in the
-//    fp32 MFMA's B layout;
+//    coefficients, one more swap gives every lane its column's scales of both groups, and the offsets already lie in
+//    the fp32 MFMA's B layout;
 //  - each scale group closes as acc += s * sum x (128 + q) on the VALU, and the offsets of both groups, (z - 128 s) *
 //    sum x, in one 32x32x2 fp32 MFMA a row block.
 // The passes are bound by instruction issue; a row's result depends only on its own activations.
@@ -75,21 +75,23 @@ template <int RB>
 __device__ __forceinline__ uint32_t stage_row() {
   return RB == 2 ? threadIdx.x >> 3 : 4 * (threadIdx.x >> 6) + ((threadIdx.x >> 3) & 3);
 }
-// That row in the input: a pointer to the lane's chunk, or, in the formats whose walk would spill the pointer (each reload
-// then waits for every load in flight), the 64-input span it begins at. Measured, block times at 33 / 128 rows of eight
-// routes over 256 experts of 2048 x 512, pointer -> span: af4g128 99 / 139 -> 89 / 130 us, Q6_K 143 / 199 -> 137 / 194;
-// af4g64 84 / 123 -> 86 / 127 (the span's address takes instructions), so the formats that don't spill keep the pointer.
+// That row in the input: a pointer to the lane's chunk, or, in the formats whose walk would spill the pointer (each
+// reload then waits for every load in flight), the 64-input span it begins at. Measured, block times at 33 / 128 rows
+// of eight routes over 256 experts of 2048 x 512, pointer -> span: af4g128 99 / 139 -> 89 / 130 us, Q6_K 143 / 199 ->
+// 137 / 194; af4g64 84 / 123 -> 86 / 127 (the span's address takes instructions), so the formats that don't spill keep
+// the pointer.
 template <uint32_t FMT>
 constexpr bool kRowSpans = FMT == SQ_FMT_AF4G128 || FMT == SQ_FMT_Q6K;
 template <uint32_t FMT>
 using RowSource = std::conditional_t<kRowSpans<FMT>, uint32_t, const uint16_t *>;
 
-// The walk of one wave over RB blocks of 32 rows: acc[b] += its 32 columns' sums, in registers 0..LIVE - 1 (LIVE 8: rows
-// 0..15 of a block). plane, high and meta: the plane tile, c0 the wave's first column of it; row: the lane's row, of the
-// workgroup's `rows`. One block stages two steps at a time (lanes 0..31 the even step's rows, 32..63 the odd one's), in
-// four half stages: one barrier and one wait for rows every two steps. Tiles of few rows run as many steps as tall ones
-// and hold little to do in each, so they were bound by that wait: 64 rows of eight routes over 256 af4g64 experts of
-// 2048 x 512, a step at a time with every wave staging and sixteen registers closed, 143 us the block; so, 115.
+// The walk of one wave over RB blocks of 32 rows: acc[b] += its 32 columns' sums, in registers 0..LIVE - 1 (LIVE 8:
+// rows 0..15 of a block). plane, high and meta: the plane tile, c0 the wave's first column of it; row: the lane's row,
+// of the workgroup's `rows`. One block stages two steps at a time (lanes 0..31 the even step's rows, 32..63 the odd
+// one's), in four half stages: one barrier and one wait for rows every two steps. Tiles of few rows run as many steps
+// as tall ones and hold little to do in each, so they were bound by that wait: 64 rows of eight routes over 256 af4g64
+// experts of 2048 x 512, a step at a time with every wave staging and sixteen registers closed, 143 us the block; so,
+// 115.
 template <uint32_t FMT, int RB, int LIVE>
 __device__ __forceinline__ void wide_walk(const MoeExpertArgs &a, const uint8_t *plane, const uint8_t *high,
                                           const uint8_t *meta, uint32_t c0, RowSource<FMT> row, uint32_t rows,
@@ -267,8 +269,8 @@ __device__ __forceinline__ void wide_walk(const MoeExpertArgs &a, const uint8_t 
       for (int b = 0; b < RB; ++b) acc[b] = mfma32_f32(sums[(32 * b + l32) * (2 * NH) + 2 * m + h], zc[m], acc[b]);
   };
 
-  // Codes come `kAhead` steps ahead into a ring of four (8-bit codes, of twice the registers: two), the meta with them or,
-  // where a unit spans the ring's four steps, a unit ahead.
+  // Codes come `kAhead` steps ahead into a ring of four (8-bit codes, of twice the registers: two), the meta with them
+  // or, where a unit spans the ring's four steps, a unit ahead.
   constexpr int kRing = F::P0 == 32 ? 2 : 4, kAhead = kRing - 1;
   constexpr bool kUnitMeta = F::UNIT == 8;
   Words w[kRing];
@@ -337,8 +339,8 @@ __device__ __forceinline__ void wide_store(const MoeExpertArgs &a, const f32x16 
       const size_t at = (size_t)(first_row + row) * a.output_size + col;
       float v = acc[b][r];
       if (a.gate_up || a.gate) {
-        const float g = a.gate_up ? bf16_to_f32(f32_to_bf16(gates[(((wave - kTensorWaves) * RB + b) * 16 + r) * 64 + lane]))
-                                  : bf16_to_f32(a.gate[at]);
+        const uint32_t place = (((wave - kTensorWaves) * RB + b) * 16 + r) * 64 + lane;
+        const float g = bf16_to_f32(a.gate_up ? f32_to_bf16(gates[place]) : a.gate[at]);
         v = bf16_to_f32(f32_to_bf16(v)) * silu(g);
       }
       a.output[at] = f32_to_bf16(v);
@@ -348,7 +350,8 @@ __device__ __forceinline__ void wide_store(const MoeExpertArgs &a, const f32x16 
 // The launch's work list in LDS: its tiles taken two of an expert at a time from the expert's first on (`single`: each
 // alone), as 2 tile + (1 if it takes the next tile too), those of two tiles first, so that the long ones do not trail.
 // Returns its entries. experts: LDS room for the tiles' experts.
-constexpr uint32_t kMaxTiles = SQ_PREFILL_TOKEN_BUDGET * 64 / 32 + SQ_MOE_WIDE_EXPERT_SLOTS + 2 * SQ_PREFILL_TOKEN_BUDGET / 32;
+constexpr uint32_t kMaxTiles =
+    SQ_PREFILL_TOKEN_BUDGET * 64 / 32 + SQ_MOE_WIDE_EXPERT_SLOTS + 2 * SQ_PREFILL_TOKEN_BUDGET / 32;
 __device__ uint32_t work_list(const MoeExpertArgs &a, uint32_t n, uint16_t *experts, uint16_t *list) {
   constexpr uint32_t kThreads = 64 * kWaves;
   __shared__ uint32_t wave_start[kWaves], wave_count[kWaves];
@@ -413,13 +416,14 @@ __device__ uint32_t work_list(const MoeExpertArgs &a, uint32_t n, uint16_t *expe
 // A workgroup runs one column group of a tile and, if it is the expert's next, the tile after it (tiles pair from the
 // expert's first on). Over a long K it takes its tiles from the work list, the tall ones first: entries go round the
 // XCDs (workgroup b runs on XCD b % 8), an entry's column groups on one XCD, whose L2 they share its rows in. Over a
-// short K, or where the routed experts hold at most 24 rows on average (most are then one tile, and the order has nothing
-// to put first), the list costs more than the order gains, and the workgroups go by tile, those of a pair's second tile
-// returning at once; tiles go round the XCDs two by two, so that those do not idle the XCDs of one parity. Measured (35B
-// layer, 1999 rows), list against tiles: gate/up of K 2048 160 against 178 us, down of K 512 136 against 121; 512 rows,
-// down of K 768 45 against 50. By rows an expert, af4g64 blocks, list against tiles: 4 (256 experts of 2048 x 512) 130
-// against 125 us, 17 (60 of 2048 x 1280) 103 against 100, 32 (128 of 2048 x 768) 157 against 167, 34 (60) 139 against 153.
-// Launches that hold shared tiles keep the list: Q8_0 with its shared slice, 64 rows, 198 against 219.
+// short K, or where the routed experts hold at most 24 rows on average (most are then one tile, and the order has
+// nothing to put first), the list costs more than the order gains, and the workgroups go by tile, those of a pair's
+// second tile returning at once; tiles go round the XCDs two by two, so that those do not idle the XCDs of one parity.
+// Measured (35B layer, 1999 rows), list against tiles: gate/up of K 2048 160 against 178 us, down of K 512 136 against
+// 121; 512 rows, down of K 768 45 against 50. By rows an expert, af4g64 blocks, list against tiles: 4 (256 experts of
+// 2048 x 512) 130 against 125 us, 17 (60 of 2048 x 1280) 103 against 100, 32 (128 of 2048 x 768) 157 against 167, 34
+// (60) 139 against 153. Launches that hold shared tiles keep the list: Q8_0 with its shared slice, 64 rows, 198 against
+// 219.
 constexpr uint32_t kListedRows = 24;
 template <uint32_t FMT>
 __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(4)))

@@ -956,22 +956,23 @@ PrefillSchedule prefill_schedule(uint32_t rows, uint32_t plane_tiles, uint32_t K
   if (7 * rounds128 < 10 * rounds256) return {128, 0, blocks128, columns, 0, 0};
   return {256, 0, blocks256, columns, 0, 0};
 }
-// The narrow tile's shape where it costs less than the wide tile that would run (prefill_schedule). Costs in microseconds,
-// fitted to Q4_K over 431 shapes of 128..2048 rows, K 256..6144 and N 512..14336 whose two costs are near each other (rms
-// 4%): what a dispatch of either takes besides (kDispatch), a 64-input step of a round of workgroups, and what a round past
-// the first adds (the narrow tile's prologue, the sums of its slices and its stores, which the first round overlaps with
-// the dispatch). The wide tile keeps what the narrow one would not win by 8%. The other formats' costs keep
-// nearly these ratios (96 x 64 a step of the 128-row tile: Q4_K 0.26, the af4 ones 0.28, Q5_K 0.26, Q6_K 0.23, 8-bit codes
-// 0.24); over the same shapes in all eight the tile chosen was never more than 2% slower than the wide one, and on average
-// 0.6% slower than the fastest of the five. Without the rounds' own cost short K took the narrow tile where it loses: 2048
-// rows of K 1024 x N 2048 26 -> 30 us (af4g64; wide again 26), 1024 of K 256 x N 4096 13 -> 21. `plane_tiles` are the
-// dispatch's own: a projection of several formats runs a dispatch for each, and each pays its own rounds (512 rows of K
-// 5120, 7168 Q4_K and 1024 Q6_K columns: 167 us halved in two dispatches, 98 on tiles
-// of their own).
+// The narrow tile's shape where it costs less than the wide tile that would run (prefill_schedule). Costs in
+// microseconds, fitted to Q4_K over 431 shapes of 128..2048 rows, K 256..6144 and N 512..14336 whose two costs are near
+// each other (rms 4%): what a dispatch of either takes besides (kDispatch), a 64-input step of a round of workgroups,
+// and what a round past the first adds (the narrow tile's prologue, the sums of its slices and its stores, which the
+// first round overlaps with the dispatch). The wide tile keeps what the narrow one would not win by 8%. The other
+// formats' costs keep nearly these ratios (96 x 64 a step of the 128-row tile: Q4_K 0.26, the af4 ones 0.28, Q5_K 0.26,
+// Q6_K 0.23, 8-bit codes 0.24); over the same shapes in all eight the tile chosen was never more than 2% slower than
+// the wide one, and on average 0.6% slower than the fastest of the five. Without the rounds' own cost short K took the
+// narrow tile where it loses: 2048 rows of K 1024 x N 2048 26 -> 30 us (af4g64; wide again 26), 1024 of K 256 x N 4096
+// 13 -> 21. `plane_tiles` are the dispatch's own: a projection of several formats runs a dispatch for each, and each
+// pays its own rounds (512 rows of K 5120, 7168 Q4_K and 1024 Q6_K columns: 167 us halved in two dispatches, 98 on
+// tiles of their own).
 PrefillNarrow prefill_narrow(uint32_t rows, uint32_t plane_tiles, uint32_t K, bool split) {
   const double steps = K / BK, kDispatch = 9.0;
   const auto rounds = [&](uint32_t r, uint32_t c) {
-    return (double)(((uint64_t)((rows + r - 1) / r) * ((plane_tiles * 64 + c - 1) / c) + kPrefillUnits - 1) / kPrefillUnits);
+    const uint64_t tiles = (uint64_t)((rows + r - 1) / r) * ((plane_tiles * 64 + c - 1) / c);
+    return (double)((tiles + kPrefillUnits - 1) / kPrefillUnits);
   };
   const PrefillSchedule sc = prefill_schedule(rows, plane_tiles, K, split);
   const double wide = sc.split       ? 0.725 * steps + 16.0
@@ -1013,8 +1014,8 @@ PrefillStream prefill_stream(uint32_t row_blocks, uint32_t column_groups, uint32
   if (steps > 2 * range) return {0, 0, 0, 0};
   return {dp, stream, range, dp + row_blocks * ((work + range - 1) / range)};
 }
-// The halves' partials are reserved wherever the 256-row tiles would halve, also where every dispatch runs the narrow tile:
-// a plan's scratch, and so what a caller's scratch accepts and refuses, does not follow the measured costs.
+// The halves' partials are reserved wherever the 256-row tiles would halve, also where every dispatch runs the narrow
+// tile: a plan's scratch, and so what a caller's scratch accepts and refuses, does not follow the measured costs.
 PrefillScratch prefill_scratch_bytes(uint32_t rows, uint32_t plane_tiles, uint32_t K) {
   if (prefill_split(rows, plane_tiles, K)) return {(uint64_t)2 * rows * ((plane_tiles + 3) / 4) * 256 * 4, 0};
   // A stream dispatch (any of the projection's, one a format, whose 256-row tiles are at most all of the

@@ -108,8 +108,9 @@ void narrow_kernel(PrefillArgs a, uint32_t epilogue) {
     float *const cs = (float *)(xs + kRowBytes);   // (s, z) or half scales of [group][column]
     // The lane's column and (32 columns) its group of a step.
     const uint32_t col = NT == 4 ? lane : c0 + (lane & 31), half = NT == 4 ? 0u : lane >> 5;
-    // Buffer resources over the tile's planes and the workgroup's own rows (32-bit lane offsets, the step's offset scalar;
-    // the extent of a whole chunk's rows would wrap from 4 GiB on, 2048 rows of K 2^20, and every load then read zeros).
+    // Buffer resources over the tile's planes and the workgroup's own rows (32-bit lane offsets, the step's offset
+    // scalar; the extent of a whole chunk's rows would wrap from 4 GiB on, 2048 rows of K 2^20, and every load then
+    // read zeros).
     const uint32_t live = min((uint32_t)BM, a.rows - row0);
     const auto planes = buffer_rsrc(seg.plane0 + (size_t)ptile * G * 64 * F::P0, G * 64 * F::P0);
     const auto metas = buffer_rsrc(seg.meta + (size_t)ptile * units * 64 * F::META, units * 64 * F::META);

@@ -362,76 +362,66 @@ __device__ __forceinline__ void row_slice(const RowBuffers<FMT, NT, MB, TB> &src
   }
 }
 
-// Adds groups first .. end - 1 of NT tensors' plane tiles to acc, as row_slice does, in one continuous stream: chunks
-// of CH groups, each chunk's loads (clamped to the last group, so every chunk issues as many) issued SETS - 1 chunks
-// ahead into a ring of SETS register sets; first is a multiple of CH and of the meta unit or lies CH-aligned inside a
-// longer one. plane[n] and high[n] point at group 0 for the lane, meta[n] at unit 0 of the lane's own column l (one
-// load per unit and tensor, spread_coefs hands each lane the columns its MFMA blocks hold). The input rows come in the
-// tile's read order
-// (16-byte chunk 4 g + c of a row: inputs 32 g + 4 c .. +3 then 32 g + 16 + 4 c .. +3), so each group of a row block
-// is one 16-byte load a lane, half the vector memory instructions of two 8-byte loads from a row in input order:
-// xrow[b] points at chunk q of group 0 of the lane's row 16 b + j.
-template <uint32_t FMT, int MB, int NT, int SETS = 2, int CH = 4>
-__device__ __forceinline__ void row_stream(const uint8_t *const (&plane)[NT], const uint8_t *const (&high)[NT],
-                                           const uint8_t *const (&meta)[NT], const uint16_t *const (&xrow)[MB],
-                                           uint32_t first, uint32_t end, float (&acc)[NT][4][MB][4]) {
+// Adds groups first .. end - 1 of a plane tile to acc, as row_slice does for one row block, in one continuous stream:
+// chunks of CH groups, each chunk's loads (clamped to the last group, so every chunk issues as many) issued a chunk
+// ahead into the other of two register sets; first is a multiple of CH and of the meta unit or lies CH-aligned inside a
+// longer one. plane and high point at group 0 for the lane, meta at unit 0 of the lane's own column l (one load a unit,
+// spread_coefs hands each lane the columns its MFMA blocks hold). The input rows come in the tile's read order (16-byte
+// chunk 4 g + c of a row: inputs 32 g + 4 c .. +3 then 32 g + 16 + 4 c .. +3), so each group is one 16-byte load a
+// lane, half the vector memory instructions of two 8-byte loads from a row in input order: xrow points at chunk q of
+// group 0 of the lane's row j.
+template <uint32_t FMT, int CH>
+__device__ __forceinline__ void row_stream(const uint8_t *plane, const uint8_t *high, const uint8_t *meta,
+                                           const uint16_t *xrow, uint32_t first, uint32_t end,
+                                           float (&acc)[1][4][1][4]) {
   using F = Fmt<FMT>;
   constexpr int SG = F::SG, UNIT = F::UNIT, MU = UNIT < CH ? CH / UNIT : 1;
   static_assert(CH % SG == 0, "a chunk holds whole scale groups");
   const uint32_t last = end - 1, chunks = (end - first + CH - 1) / CH;
   const CodeConstants cc = make_code_constants();
   const uint32_t hshift = row_high_shift<FMT>(threadIdx.x & 63);
-  u32x4 xv[SETS][MB][CH];
-  RowGroup<FMT> codes[SETS][NT][CH];
-  MetaWords own[SETS][NT][MU];
+  u32x4 xv[2][CH];
+  RowGroup<FMT> codes[2][CH];
+  MetaWords own[2][MU];
   const auto issue = [&](uint32_t c, int set) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < CH; ++u) {
       const uint32_t g = min(first + c * CH + u, last);
-#pragma unroll
-      for (int b = 0; b < MB; ++b) xv[set][b][u] = *(const u32x4 *)(xrow[b] + (size_t)g * 32);
-#pragma unroll
-      for (int n = 0; n < NT; ++n) codes[set][n][u] = load_row_group<FMT>(plane[n], high[n], g);
+      xv[set][u] = *(const u32x4 *)(xrow + (size_t)g * 32);
+      codes[set][u] = load_row_group<FMT>(plane, high, g);
     }
 #pragma unroll
     for (int m = 0; m < MU; ++m) {
       const uint32_t unit = min((first + c * CH) / UNIT + m, last / UNIT);
-#pragma unroll
-      for (int n = 0; n < NT; ++n) own[set][n][m] = load_meta<FMT>(meta[n] + (size_t)unit * 64 * F::META);
+      own[set][m] = load_meta<FMT>(meta + (size_t)unit * 64 * F::META);
     }
   };
-  f32x4 C[NT][4][MB], C2[NT][4][MB], S[MB], S2[MB];
-  u32x4 lo[NT][4], hi[NT][4];
+  f32x4 C[1][4][1], C2[1][4][1], S[1], S2[1];
+  u32x4 lo[1][4], hi[1][4];
   const int j = threadIdx.x & 15;
   const auto compute = [&](uint32_t c, int set) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < CH; ++u) {
       const uint32_t g = first + c * CH + u;
       if (g < end) {
-        u32x4 x[MB];
-#pragma unroll
-        for (int b = 0; b < MB; ++b) x[b] = xv[set][b][u];
-#pragma unroll
-        for (int n = 0; n < NT; ++n) row_operands<FMT>(codes[set][n][u], hshift, cc, lo[n], hi[n]);
-        row_group_mfma<FMT, MB, NT>(x, lo, hi, u % SG == 0, C, C2, S, S2);
+        const u32x4 x[1] = {xv[set][u]};
+        row_operands<FMT>(codes[set][u], hshift, cc, lo[0], hi[0]);
+        row_group_mfma<FMT, 1, 1>(x, lo, hi, u % SG == 0, C, C2, S, S2);
         if ((u + 1) % SG == 0) {
-          MetaWords unit[NT];
-#pragma unroll
-          for (int n = 0; n < NT; ++n) unit[n] = own[set][n][UNIT < CH ? u / UNIT : 0];
-          CloseCoef k[NT][4];
-          spread_coefs<FMT, NT>(unit, g, j, k);
-          row_group_close<FMT, MB, NT>(k, C, C2, S, S2, acc);
+          const MetaWords unit[1] = {own[set][UNIT < CH ? u / UNIT : 0]};
+          CloseCoef k[1][4];
+          spread_coefs<FMT, 1>(unit, g, j, k);
+          row_group_close<FMT, 1, 1>(k, C, C2, S, S2, acc);
         }
       }
       __builtin_amdgcn_sched_barrier(0);
     }
   };
+  issue(0, 0);
+  for (uint32_t c = 0; c < chunks; c += 2) {
 #pragma unroll
-  for (int c = 0; c < SETS - 1; ++c) issue(c, c);
-  for (uint32_t c = 0; c < chunks; c += SETS) {
-#pragma unroll
-    for (int k = 0; k < SETS; ++k) {
-      issue(c + k + SETS - 1, (k + SETS - 1) % SETS);
+    for (int k = 0; k < 2; ++k) {
+      issue(c + k + 1, 1 - k);
       __builtin_amdgcn_sched_barrier(0);
       compute(c + k, k);
     }
