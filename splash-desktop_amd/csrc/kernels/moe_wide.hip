@@ -16,7 +16,10 @@
 //    the fp32 MFMA's B layout;
 //  - each scale group closes as acc += s * sum x (128 + q) on the VALU, and the offsets of both groups, (z - 128 s) *
 //    sum x, in one 32x32x2 fp32 MFMA a row block.
-// The passes are bound by instruction issue; a row's result depends only on its own activations.
+// The passes are bound by instruction issue (VALU issue 59% of the gate/up dispatch above) and, where tiles hold few rows,
+// by their steps' waits. Of the instances (128 registers) all but af4g64's spill, 28 to 128 bytes a lane; in the hot loops
+// only Q5_K's and Q6_K's over 64 rows (two and seven reloads or stores every four steps). A row's result depends only on
+// its own activations.
 #include <type_traits>
 
 #include "kernels.hpp"

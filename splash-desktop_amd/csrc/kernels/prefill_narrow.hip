@@ -8,7 +8,8 @@
 // of K: measured, Q4_K, wide -> narrow, N 5120 x K 6144 at 77 / 256 / 512 rows 98 / 100 / 102 -> 22 / 31 / 64 us, N
 // 4096 x K 14336 at 48 / 256 / 512 rows 223 / 226 / 227 -> 32 / 54 / 104, N 1024 x K 4096 at 1024 rows 68 -> 20; N
 // 14336 x K 4096 at 512 rows would go 87 -> 129 (prefill_narrow draws the line). Bound by instruction issue (the
-// dequantisation) and the waves' LDS traffic; sixteen waves a workgroup measured no faster. Per step a wave
+// dequantisation) where the chip is full, by the waves' step chains where it is not; sixteen waves a workgroup measured
+// no faster. Per step a wave
 //  - brings the rows' 128 bytes as they lie (eight lanes a row, whole cache lines; fragment loads straight from memory
 //    would touch a line a lane) into registers a step ahead, and turns them into the MFMA's layout through its own LDS
 //    (the swizzle of chunk_slot, conflict-free both ways);
