@@ -967,7 +967,9 @@ PrefillSchedule prefill_schedule(uint32_t rows, uint32_t plane_tiles, uint32_t K
 // narrow tile where it loses: 2048 rows of K 1024 x N 2048 26 -> 30 us (af4g64; wide again 26), 1024 of K 256 x N 4096
 // 13 -> 21. `plane_tiles` are the dispatch's own: a projection of several formats runs a dispatch for each, and each
 // pays its own rounds (512 rows of K 5120, 7168 Q4_K and 1024 Q6_K columns: 167 us halved in two dispatches, 98 on
-// tiles of their own).
+// tiles of their own). Which wide tile would run is prefill_split's and prefill_schedule's to say, by their own earlier
+// estimates of the same costs (a 128-row tile 0.7 of a 256-row one, here 0.64; a halved one steps / 2 + 8, here 0.47
+// steps + 10): prefill_split sizes the scratch, so it does not move with these.
 PrefillNarrow prefill_narrow(uint32_t rows, uint32_t plane_tiles, uint32_t K, bool split) {
   const double steps = K / BK, kDispatch = 9.0;
   const auto rounds = [&](uint32_t r, uint32_t c) {

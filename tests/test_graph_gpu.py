@@ -90,6 +90,16 @@ def test_graph_halved_prefill():
     linear_case(plan, proj, n, rows, k, rng)
 
 
+@pytest.mark.parametrize("static", [False, True])
+def test_graph_narrow_prefill(static):
+    rng = np.random.default_rng(96)
+    n, k, rows = 1088, 2048, 100
+    w = make_weights(rng, oracle.FMT_Q4K, n, k)
+    proj = sq.projection(w.segment())
+    assert prefill_tile(rows, n, k) == "64x32"
+    linear_case(sq.plan_for(sq.prefill_workload(n, k, rows), proj), proj, n, rows, k, rng, static=static)
+
+
 def test_graph_stream_prefill():
     rng = np.random.default_rng(93)
     n, k, rows = 24576, 1280, 1024
