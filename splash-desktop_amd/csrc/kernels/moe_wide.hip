@@ -94,7 +94,7 @@ using RowSource = std::conditional_t<kRowSpans<FMT>, uint32_t, const uint16_t *>
 // one's), in four half stages: one barrier and one wait for rows every two steps. Tiles of few rows run as many steps
 // as tall ones and hold little to do in each, so they were bound by that wait: 64 rows of eight routes over 256 af4g64
 // experts of 2048 x 512, a step at a time with every wave staging and sixteen registers closed, 143 us the block; so,
-// 115.
+// 115 to 119. (Four steps at a time up to 16 rows: 1.01 x that; rings of six or eight steps of codes 1.08 and 1.17.)
 template <uint32_t FMT, int RB, int LIVE>
 __device__ __forceinline__ void wide_walk(const MoeExpertArgs &a, const uint8_t *plane, const uint8_t *high,
                                           const uint8_t *meta, uint32_t c0, RowSource<FMT> row, uint32_t rows,
